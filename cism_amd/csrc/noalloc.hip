@@ -52,58 +52,172 @@ struct FGrid {
     long long nn;
 };
 
-// one lane per node (grid-stride): r = A x - b on owned active rows, 0 elsewhere; the
-// 27 slots summed in indxA order as the reference's row product (pcg:2607-2645), so the
-// vector equals the context entry point's bit for bit.  part[2 * block + {0, 1}] =
-// the block's |r|^2 and |b|^2 over owned active rows, in a fixed order.
-__global__ __launch_bounds__(NOALLOC_THREADS) void k_resvec_fortran(
+// r = A x - b on owned active rows, 0 elsewhere; the 27 slots summed in indxA order as the
+// reference's row product (pcg:2607-2645), so the vector equals the context entry point's bit
+// for bit.  part[2 * block + {0, 1}] = the block's |r|^2 and |b|^2 over owned active rows, in a
+// fixed order.
+//
+// Bound: one read of the four blocks, 864 of the 912 bytes a node needs.  In the Fortran layout
+// a node's 27 coefficients of a block are 216 contiguous bytes, so lanes that walk their own
+// rows touch 64 lines per load and fetch every line again for most of the 27 slots (2.9 ms,
+// 0.78 TB/s, at 503 x 453 x 11).  Here a workgroup is one wave and takes tiles of 64 nodes: it
+// loads the tile's two blocks of one row (Auu, Auv, then Avu, Avv) as contiguous runs into
+// registers, passes them through LDS (27.6 KB, four or five waves per CU; the stride of 27
+// doubles is odd, so the row reads are conflict-free) and loads the next pair while it sums
+// this one: 110 KB per CU in flight.  0.50 ms at that size with three quarters of the columns
+// active (21.7 -> 13.5 us a call at 34 x 34 x 10).  A tile without an owned active node is
+// not read.
+// W doubles per load: 2 when the four blocks are 16-byte aligned (a tile starts at a
+// multiple of 13,824 bytes), else 1.
+template <int W>
+struct RowPair {
+    static constexpr int N = (27 * 64 / W + 63) / 64;   // loads per lane and block
+    double a[N][W], b[N][W];
+};
+
+template <int W>
+__device__ __forceinline__ void pair_load(RowPair<W> &R, const double *__restrict__ A, const double *__restrict__ B,
+                                          long long q0, int count, int lane) {
+    typedef double vec __attribute__((ext_vector_type(W)));
+    const double *pa = A + 27 * q0, *pb = B + 27 * q0;
+#pragma unroll
+    for (int t = 0; t < RowPair<W>::N; ++t) {
+        const int e = (t * 64 + lane) * W;
+        if (e + W <= count) {
+            const vec va = *reinterpret_cast<const vec *>(pa + e), vb = *reinterpret_cast<const vec *>(pb + e);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                R.a[t][w] = va[w];
+                R.b[t][w] = vb[w];
+            }
+        } else if (e < count) {   // the odd last value of the grid
+            R.a[t][0] = pa[e];
+            R.b[t][0] = pb[e];
+        }
+    }
+}
+
+template <>
+__device__ __forceinline__ void pair_load<1>(RowPair<1> &R, const double *__restrict__ A,
+                                             const double *__restrict__ B, long long q0, int count, int lane) {
+    const double *pa = A + 27 * q0, *pb = B + 27 * q0;
+#pragma unroll
+    for (int t = 0; t < RowPair<1>::N; ++t) {
+        const int e = t * 64 + lane;
+        if (e < count) {
+            R.a[t][0] = pa[e];
+            R.b[t][0] = pb[e];
+        }
+    }
+}
+
+// the pair to LDS, slot-minor as in memory; a lane's row is then S[27 * lane ..]
+template <int W>
+__device__ __forceinline__ void pair_stage(const RowPair<W> &R, double *__restrict__ SA, double *__restrict__ SB,
+                                           int lane) {
+#pragma unroll
+    for (int t = 0; t < RowPair<W>::N; ++t) {
+        const int e = (t * 64 + lane) * W;
+        if (e < 27 * 64)
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                SA[e + w] = R.a[t][w];
+                SB[e + w] = R.b[t][w];
+            }
+    }
+}
+
+template <int W>
+__global__ __launch_bounds__(64) void k_resvec_fortran(
     FGrid g, const int32_t *__restrict__ av, const double *__restrict__ Auu, const double *__restrict__ Auv,
     const double *__restrict__ Avu, const double *__restrict__ Avv, const double *__restrict__ bu,
     const double *__restrict__ bv, const double *__restrict__ xu, const double *__restrict__ xv,
     double *__restrict__ ru, double *__restrict__ rv, double *__restrict__ part) {
-    double acc[2] = {0.0, 0.0};
-    const long long stride = (long long)gridDim.x * blockDim.x;
+    __shared__ alignas(16) double SA[27 * 64], SB[27 * 64];
+    const int lane = threadIdx.x;
     const long long cst = g.nz, rst = (long long)g.nz * g.sx;
-    for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
-        double r0 = 0.0, r1 = 0.0;
-        if (i >= g.ilo && i <= g.ihi && j >= g.jlo && j <= g.jhi && av[col]) {
-            double su = 0.0, sv = 0.0;
-            const double *au = Auu + 27 * q, *auv = Auv + 27 * q, *avu = Avu + 27 * q, *avv = Avv + 27 * q;
+    const int ntiles = (int)((g.nn + 63) / 64);
+    double acc[2] = {0.0, 0.0};
+    RowPair<W> R = {};
+    // this lane's node of a tile: whether it has a row, and its level
+    auto row_of = [&](int tile, int &k) {
+        const long long q = (long long)tile * 64 + lane;
+        if (q >= g.nn) return false;
+        const int qi = (int)q, col = qi / g.nz;   // grids end at 2^30 nodes
+        k = qi - col * g.nz;
+        const int j = col / g.sx, i = col - j * g.sx;
+        return i >= g.ilo && i <= g.ihi && j >= g.jlo && j <= g.jhi && av[col] != 0;
+    };
+    auto count_of = [&](int tile) {
+        const long long left = g.nn - (long long)tile * 64;
+        return (int)(left < 64 ? left : 64) * 27;
+    };
+    // the next tile with a row from `tile` on; the rowless ones before it are written here
+    bool row = false;
+    int k = 0;
+    auto find = [&](int tile) {
+        for (; tile < ntiles; tile += gridDim.x) {
+            row = row_of(tile, k);
+            if (__any(row)) break;
+            const long long q = (long long)tile * 64 + lane;
+            if (q < g.nn) {
+                ru[q] = 0.0;
+                rv[q] = 0.0;
+            }
+        }
+        return tile;
+    };
+    // one component's row product from the staged pair, slots in indxA order
+    auto product = [&](long long q, bool act, int kk) {
+        double s = 0.0;
+        if (act) {
 #pragma unroll
             for (int m = 0; m < 27; ++m) {
                 const int iA = m % 3 - 1, jA = (m / 3) % 3 - 1, kA = m / 9 - 1;
-                if (k + kA < 0 || k + kA >= g.nz) continue;
+                if (kk + kA < 0 || kk + kA >= g.nz) continue;
                 const long long qn = q + kA + iA * cst + jA * rst;
-                const double x0 = xu[qn], x1 = xv[qn];
-                su = su + au[m] * x0 + auv[m] * x1;
-                sv = sv + avu[m] * x0 + avv[m] * x1;
+                s = s + SA[27 * lane + m] * xu[qn] + SB[27 * lane + m] * xv[qn];
             }
-            r0 = su - bu[q];
-            r1 = sv - bv[q];
-            acc[0] += r0 * r0 + r1 * r1;
-            acc[1] += bu[q] * bu[q] + bv[q] * bv[q];
         }
-        ru[q] = r0;
-        rv[q] = r1;
+        return s;
+    };
+    int tile = find(blockIdx.x);
+    if (tile < ntiles) pair_load<W>(R, Auu, Auv, (long long)tile * 64, count_of(tile), lane);
+    while (tile < ntiles) {
+        const long long q = (long long)tile * 64 + lane;
+        const bool act = row;
+        const int kk = k;
+        pair_stage<W>(R, SA, SB, lane);
+        pair_load<W>(R, Avu, Avv, (long long)tile * 64, count_of(tile), lane);
+        __syncthreads();
+        const double su = product(q, act, kk);
+        __syncthreads();
+        pair_stage<W>(R, SA, SB, lane);
+        const int next = find(tile + gridDim.x);
+        if (next < ntiles) pair_load<W>(R, Auu, Auv, (long long)next * 64, count_of(next), lane);
+        __syncthreads();
+        const double sv = product(q, act, kk);
+        __syncthreads();
+        double r0 = 0.0, r1 = 0.0;
+        if (act) {
+            const double b0 = bu[q], b1 = bv[q];
+            r0 = su - b0;
+            r1 = sv - b1;
+            acc[0] += r0 * r0 + r1 * r1;
+            acc[1] += b0 * b0 + b1 * b1;
+        }
+        if (q < g.nn) {
+            ru[q] = r0;
+            rv[q] = r1;
+        }
+        tile = next;
     }
-    // fixed-order block reduction: waves by shuffles, then wave 0 over the waves
-    __shared__ double red[NOALLOC_THREADS / 64][2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         double s = acc[c];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        if (lane == 0) red[wave][c] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        double s = 0.0;
-        for (int w = 0; w < NOALLOC_THREADS / 64; ++w) s += red[w][threadIdx.x];
-        part[2 * blockIdx.x + threadIdx.x] = s;
+        if (lane == 0) part[2 * blockIdx.x + c] = s;
     }
 }
 
@@ -167,11 +281,13 @@ extern "C" int cism_compute_residual_vector_3d_noalloc(int nx, int ny, int nz, i
     g.jlo = (periodic ? 3 : 2) - 1;
     g.ihi = nx - 3;
     g.jhi = ny - 3;
-    long long nb = (nn + NOALLOC_THREADS - 1) / NOALLOC_THREADS;
+    long long nb = (nn + 63) / 64;   // one wave per tile of 64 nodes
     if (nb > NOALLOC_BLOCKS) nb = NOALLOC_BLOCKS;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_resvec_fortran, dim3((unsigned)nb), dim3(NOALLOC_THREADS), 0, s, g, active_vertex, Auu,
-                       Auv, Avu, Avv, bu, bv, uvel, vvel, resid_u, resid_v, part);
+    // 16-byte loads of the blocks only when the caller's arrays allow them
+    const bool wide = (((uintptr_t)Auu | (uintptr_t)Auv | (uintptr_t)Avu | (uintptr_t)Avv) & 15) == 0;
+    hipLaunchKernelGGL(wide ? k_resvec_fortran<2> : k_resvec_fortran<1>, dim3((unsigned)nb), dim3(64), 0, s, g,
+                       active_vertex, Auu, Auv, Avu, Avv, bu, bv, uvel, vvel, resid_u, resid_v, part);
     hipLaunchKernelGGL(k_resvec_norms, dim3(1), dim3(NOALLOC_THREADS), 0, s, (int)nb, part, norms);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
