@@ -156,6 +156,9 @@ struct cism_ctx {
     int as_ok;
     // reductions
     double *partials;
+    // the matvecs' dot partials, 2 per node block: the FP64 ones, and the FP32 ones in the
+    // order of xcd_slot, a buffer of their own whose places past the last block stay zero
+    double *mpart, *mpart32;
     double *red_groups;   // the first pass of a two-pass reduction (RED_GROUPS x CISM_MAX_NV)
     DevScal *sc;
     DevScal *sc_host;   // pinned mirror
@@ -334,20 +337,35 @@ inline int nblocks_for(long long n, int block = CISM_BLOCK) {
     long long b = (n + block - 1) / block;
     return (int)(b < 1 ? 1 : b);
 }
-// XCD-aware launch of the FP32 symmetric matvec: workgroups are dealt round-robin
-// to the 8 XCDs, so a grid of xcd_blocks_for(n) blocks (a multiple of 8 chunks) lets
-// XCD x take chunks x, x+8, x+16, ... of CISM_XCD_CHUNK consecutive node blocks; the
-// neighbours a node reads from the row before it were then read by the same XCD
-// moments earlier and sit in its L2
+// XCD-aware launch of the symmetric matvecs: workgroups are dealt round-robin to the 8
+// XCDs, so a grid of 8 * rounds * chunk blocks lets XCD x take chunks x, x+8, x+16, ... of
+// `chunk` consecutive node blocks; the neighbours a node reads from the row before it were
+// then read by the same XCD moments earlier and sit in its L2.  At most CISM_XCD_CHUNK
+// blocks a chunk, and the same number of chunks for every XCD: with chunks of 128 whatever
+// the size, a grid of up to 128 blocks ran on one XCD and one of 2,180 gave some XCDs three
+// chunks and others two.
 #define CISM_XCD_CHUNK 128
-inline int xcd_blocks_for(long long n) {
+inline int xcd_rounds_for(long long n) {
     const long long per = 8LL * CISM_XCD_CHUNK;
-    return (int)((nblocks_for(n) + per - 1) / per * per);
+    return (int)((nblocks_for(n) + per - 1) / per);
 }
-__device__ inline long long xcd_block() {
+inline int xcd_chunk_for(long long n) {
+    const int per = 8 * xcd_rounds_for(n);
+    return (nblocks_for(n) + per - 1) / per;
+}
+inline int xcd_blocks_for(long long n) { return 8 * xcd_rounds_for(n) * xcd_chunk_for(n); }
+__device__ inline long long xcd_block(unsigned chunk) {
     const unsigned b = blockIdx.x, x = b & 7u, k = b >> 3;
-    return ((long long)(k / CISM_XCD_CHUNK) * 8 + x) * CISM_XCD_CHUNK + (k % CISM_XCD_CHUNK);
+    return (long long)(((k / chunk) * 8 + x) * chunk + k % chunk);
 }
+// partial sums of the FP32 matvec: node block lb's place in the order in which its sums are
+// added (chunks of CISM_XCD_CHUNK blocks dealt to the XCDs), of xcd_slots_for(n) places;
+// the places past the last node block hold zeros
+__device__ inline long long xcd_slot(long long lb) {
+    const unsigned l = (unsigned)lb, c = l / CISM_XCD_CHUNK;
+    return ((c >> 3) * CISM_XCD_CHUNK + l % CISM_XCD_CHUNK) * 8 + (c & 7u);
+}
+inline int xcd_slots_for(long long n) { return 8 * CISM_XCD_CHUNK * xcd_rounds_for(n); }
 
 inline int red_blocks_for(long long n) {
     long long b = (n + CISM_BLOCK - 1) / CISM_BLOCK;
@@ -388,7 +406,8 @@ enum ReduceMode {
     RED_ERR,            // err = sqrt(s0)/L2_rhs
     RED_MAX             // max instead of sum (sums[c] = max)
 };
-int launch_reduce(cism_ctx *c, int nb, int nv, int mode);
+// part = null: of c->partials
+int launch_reduce(cism_ctx *c, int nb, int nv, int mode, const double *part = nullptr);
 
 int launch_matvec64(cism_ctx *c, const double *A, const double *x, double *y);
 int launch_halo_vec(cism_ctx *c, double *v);      // 2-component vector

@@ -158,27 +158,28 @@ __global__ void k_reduce_final(const double *__restrict__ groups, int mode, DevS
 }
 
 template <int NV>
-static void launch_reduce2(cism_ctx *c, int nb, int mode, double *out = nullptr) {
-    hipLaunchKernelGGL(k_reduce_groups<NV>, dim3(RED_GROUPS), dim3(CISM_BLOCK), 0, c->stream, c->partials, nb,
-                       mode, c->red_groups);
+static void launch_reduce2(cism_ctx *c, int nb, int mode, const double *part, double *out = nullptr) {
+    hipLaunchKernelGGL(k_reduce_groups<NV>, dim3(RED_GROUPS), dim3(CISM_BLOCK), 0, c->stream, part, nb, mode,
+                       c->red_groups);
     hipLaunchKernelGGL(k_reduce_final<NV>, dim3(1), dim3(64), 0, c->stream, c->red_groups, mode, c->sc, out);
 }
 
 // sums of NV values per block of the partials into out[0..NV), nothing else
 template <int NV>
 static int launch_reduce_to(cism_ctx *c, int nb, double *out) {
-    launch_reduce2<NV>(c, nb, RED_SUMS, out);
+    launch_reduce2<NV>(c, nb, RED_SUMS, c->partials, out);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
 }
 
-int launch_reduce(cism_ctx *c, int nb, int nv, int mode) {
-    if (nv == 1) launch_reduce2<1>(c, nb, mode);
-    else if (nv == 2) launch_reduce2<2>(c, nb, mode);
-    else if (nv == 4) launch_reduce2<4>(c, nb, mode);
-    else if (nv == 5) launch_reduce2<5>(c, nb, mode);
+int launch_reduce(cism_ctx *c, int nb, int nv, int mode, const double *part) {
+    if (!part) part = c->partials;
+    if (nv == 1) launch_reduce2<1>(c, nb, mode, part);
+    else if (nv == 2) launch_reduce2<2>(c, nb, mode, part);
+    else if (nv == 4) launch_reduce2<4>(c, nb, mode, part);
+    else if (nv == 5) launch_reduce2<5>(c, nb, mode, part);
     else
-        hipLaunchKernelGGL(k_reduce, dim3(1), dim3(RED_THREADS), 0, c->stream, c->partials, nb, nv, mode, c->sc);
+        hipLaunchKernelGGL(k_reduce, dim3(1), dim3(RED_THREADS), 0, c->stream, part, nb, nv, mode, c->sc);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
 }
@@ -200,7 +201,7 @@ template <> struct Vec2<double> { using t = double2; };
 template <typename T>
 struct MatFull {   // all 27 slots stored (aidx)
     static constexpr bool xcd = false;
-    static constexpr bool node_partials = false;
+    static constexpr bool slots = false;
     const T *A;
     __device__ inline void blocks(long long q, int m, long long qn, T &uu, T &uv, T &vu, T &vv) const {
         (void)qn;
@@ -215,7 +216,7 @@ struct MatFull {   // all 27 slots stored (aidx)
 
 struct MatSym32 {   // FP32 symmetric storage (sidx); matvec launched XCD-aware
     static constexpr bool xcd = true;
-    static constexpr bool node_partials = false;   // partials in launch order
+    static constexpr bool slots = true;   // partials in the order of xcd_slot
     const float *A;
     __device__ inline void blocks(long long q, int m, long long qn, float &uu, float &uv, float &vu,
                                   float &vv) const {
@@ -239,12 +240,12 @@ struct MatSym32 {   // FP32 symmetric storage (sidx); matvec launched XCD-aware
 // FP64 symmetric storage (s64idx) of an exactly symmetric FP64 matrix: the same products
 // as MatFull on it, bit for bit, from 448 instead of 864 stored bytes per node.  XCD: the
 // matvec's launch order (see xcd_block); its dot partials keep the node-block order of the
-// plain launch either way (partial_block), so every sum is the one MatFull gives.
+// plain launch either way, so every sum is the one MatFull gives.
 #define CISM_SYM64_XCD true
 template <bool XCD>
 struct MatSym64 {
     static constexpr bool xcd = XCD;
-    static constexpr bool node_partials = true;
+    static constexpr bool slots = false;   // partials in node-block order
     const double *A;
     __device__ inline void blocks(long long q, int m, long long qn, double &uu, double &uv, double &vu,
                                   double &vv) const {
@@ -329,8 +330,10 @@ int launch_matvec64(cism_ctx *c, const double *A, const double *x, double *y) {
 //   NDOT = 2: s0 = (r, x), s1 = (y, x)  [Chron-Gear (r, z), (Az, z)]
 // One lane per node, one pass over the grid; block partials go to a second
 // deterministic pass (k_reduce).
+// FP64, 163 x 163 x 21: 74.2 us with chunks of 128 blocks, 64.1 us with chunks of equal number
+// for every XCD (xcd_chunk_for); 35 x 35 x 10, 46 blocks, 5.9 -> 5.7 us.
 template <typename T, int NDOT, typename M>
-__global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, const M A,
+__global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, unsigned chunk, const M A,
                                                             const int32_t *__restrict__ av,
                                                             const T *__restrict__ x, T *__restrict__ y,
                                                             const T *__restrict__ r,
@@ -339,7 +342,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, const M A
     double acc[NDOT];
 #pragma unroll
     for (int c = 0; c < NDOT; ++c) acc[c] = 0.0;
-    const long long lb = M::xcd ? xcd_block() : (long long)blockIdx.x;
+    const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;
+    // a padding block of an XCD grid has no place
+    if (M::xcd && lb * blockDim.x >= g.nn) return;
     const long long q = lb * blockDim.x + threadIdx.x;
     if (q < g.nn) {
         const int k = (int)(q % g.nz);
@@ -360,21 +365,22 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, const M A
             }
         }
     }
-    // node_partials: the partials of node block lb sit where the plain launch puts them
-    block_reduce_store<NDOT>(acc, partials, M::node_partials ? lb : -1);
+    block_reduce_store<NDOT>(acc, partials, M::slots ? xcd_slot(lb) : lb);
 }
 
 // r = b - A x on the full grid (A x = 0 off owned active rows), s0 = (r, r) over
 // owned nodes.  halo_r: the halo takes the periodic image of r afterwards
 // (Chron-Gear, pcg:1592-1595), computed here from the image row directly.
 template <typename T, typename M>
-__global__ __launch_bounds__(CISM_BLOCK) void k_residual(GridDev g, const M A,
+__global__ __launch_bounds__(CISM_BLOCK) void k_residual(GridDev g, unsigned chunk, const M A,
                                                          const int32_t *__restrict__ av,
                                                          const T *__restrict__ x,
                                                          const T *__restrict__ b, T *__restrict__ r,
                                                          int halo_r, double *__restrict__ partials) {
     double acc[1] = {0.0};
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;   // as the matvec
+    if (M::xcd && lb * blockDim.x >= g.nn) return;
+    const long long q = lb * blockDim.x + threadIdx.x;
     if (q < g.nn) {
         const int k = (int)(q % g.nz);
         const long long col = q / g.nz;
@@ -398,7 +404,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_residual(GridDev g, const M A,
         store2<T>(r, q, ru, rv);
         if (own) acc[0] = (double)ru * ru + (double)rv * rv;
     }
-    block_reduce_store<1>(acc, partials);
+    block_reduce_store<1>(acc, partials, lb);
 }
 
 // s0 = (a, b) over owned nodes (global_sum_staggered_3d_real8, pcg:2333-2379)
@@ -1058,9 +1064,9 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     const GridDev &g = c->g;
     const int nb = red_blocks_for(g.nn), nbm = nblocks_for(g.nn), nb2 = nblocks_for(2 * g.nn);
     const int nbv = M::xcd ? xcd_blocks_for(g.nn) : nbm;   // matvec grid
-    // partials of a matvec: one per launched block, or per node block (node_partials; the
-    // padding blocks of an XCD grid, past the nodes, are left out of the sums)
-    const int nbr = M::xcd && !M::node_partials ? nbv : nbm;
+    const unsigned chunk = xcd_chunk_for(g.nn);
+    const int nbr = M::slots ? xcd_slots_for(g.nn) : nbm;   // partials of a matvec
+    double *mpart = M::slots ? c->mpart32 : c->mpart;
     const long long np = g.npad;
     // an inner solve (check = 1) whose residual becomes exactly zero has converged; the
     // reference recurrences would divide 0 by 0 there
@@ -1093,7 +1099,7 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
         // the true residual every fifth iteration, up to the synchronization that reads it
         TimerRange r_c("pcg_matmult_resid", c->stream, true);
         if (check == 0) {
-            hipLaunchKernelGGL((k_residual<T, M>), dim3(nbm), dim3(CISM_BLOCK), 0, c->stream, g, A,
+            hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A,
                                c->av, v.x, v.b, v.r, chrongear, c->partials);
             CISM_TRY(launch_reduce(c, nbm, 1, RED_ERR));
         } else if (chrongear && precond >= 2) {
@@ -1118,7 +1124,7 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     if (!chrongear) {
         // pcg:253-304: halo x, r = b - A x (no halo on r)
         CISM_TRY((launch_halo_t<T, false>(c, v.x)));
-        hipLaunchKernelGGL((k_residual<T, M>), dim3(nbm), dim3(CISM_BLOCK), 0, c->stream, g, A, c->av,
+        hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
                            v.x, v.b, v.r, 0, c->partials);
         for (int n = 1; n <= maxiters && !done; ++n) {
             CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
@@ -1129,8 +1135,8 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
                                v.d, c->sc);
             CISM_TRY((launch_halo_t<T, false>(c, v.d)));
             hipLaunchKernelGGL((k_matvec_dots<T, 1, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g,
-                               A, c->av, v.d, v.q, (const T *)nullptr, c->partials);
-            CISM_TRY(launch_reduce(c, nbr, 1, RED_STD_ETA2));
+                               chunk, A, c->av, v.d, v.q, (const T *)nullptr, mpart);
+            CISM_TRY(launch_reduce(c, nbr, 1, RED_STD_ETA2, mpart));
             hipLaunchKernelGGL(k_std_xr<T>, dim3(nb2), dim3(CISM_BLOCK), 0, c->stream, 2 * g.nn, v.d,
                                v.q, v.x, v.r, c->sc);
             if (n % 5 == 0) {
@@ -1143,20 +1149,20 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
         // x_zero the caller has set x = 0 and r = b (halo entries included).
         if (!x_zero) {
             CISM_TRY((launch_halo_t<T, false>(c, v.x)));
-            hipLaunchKernelGGL((k_residual<T, M>), dim3(nbm), dim3(CISM_BLOCK), 0, c->stream, g, A, c->av,
+            hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
                                v.x, v.b, v.r, 1, c->partials);
         }
         CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
-        hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, A,
-                           c->av, v.z, v.Az, v.r, c->partials);
-        CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_FIRST));
+        hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk,
+                           A, c->av, v.z, v.Az, v.r, mpart);
+        CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_FIRST, mpart));
         // with the SIA preconditioner the update also forms the next z
         CISM_TRY(launch_cg_update<T>(c, precond, v, 1));
         for (int n = 2; n <= maxiters && !done; ++n) {
             if (precond < 2) CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
             hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream,
-                               g, A, c->av, v.z, v.Az, v.r, c->partials);
-            CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_ITER));
+                               g, chunk, A, c->av, v.z, v.Az, v.r, mpart);
+            CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_ITER, mpart));
             CISM_TRY(launch_cg_update<T>(c, precond, v, 0, check == 1 && n % 5 == 0));
             if (n % 5 == 0) CISM_TRY(check_conv(n, done));
         }
@@ -1295,7 +1301,7 @@ int solver_mixed(cism_ctx *c, int precond, int maxiters, double tol, double inne
             CISM_TRY(launch_halo_vec(c, c->x));
             if (c->a64_valid) {
                 hipLaunchKernelGGL((k_residual<double, MatFull<double>>), dim3(nblocks_for(g.nn)),
-                                   dim3(CISM_BLOCK), 0, c->stream, g, MatFull<double>{c->A}, c->av, c->x, c->b,
+                                   dim3(CISM_BLOCK), 0, c->stream, g, 1u, MatFull<double>{c->A}, c->av, c->x, c->b,
                                    c->r, 1, c->partials);
                 CISM_TRY(launch_reduce(c, nblocks_for(g.nn), 1, RED_SUMS));
                 hipLaunchKernelGGL(k_save_scale, dim3(1), dim3(1), 0, c->stream, c->sc, 0);
@@ -1437,7 +1443,7 @@ int column_scale_device(cism_ctx *c, double *out) {
     const long long ncol = (long long)g.sx * g.sy;
     CISM_TRY(launch_halo_vec(c, c->x));
     hipLaunchKernelGGL((k_residual<double, MatFull<double>>), dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0,
-                       c->stream, g, MatFull<double>{c->A}, c->av, c->x, c->b, c->r, 1, c->partials);
+                       c->stream, g, 1u, MatFull<double>{c->A}, c->av, c->x, c->b, c->r, 1, c->partials);
     hipLaunchKernelGGL(k_colscale, dim3(nblocks_for(2 * ncol)), dim3(CISM_BLOCK), 0, c->stream, g, c->A,
                        c->av, c->x, c->b, c->r, out);
     HIP_TRY(hipGetLastError());
@@ -1649,21 +1655,22 @@ int anderson_step(cism_ctx *c, int m, double *fnorm) {
 int launch_cg_matvec(cism_ctx *c, int which) {
     const GridDev &g = c->g;
     const int nb = nblocks_for(g.nn);
+    const unsigned chunk = xcd_chunk_for(g.nn);
     if (which == 1)
         hipLaunchKernelGGL((k_matvec_dots<float, 2, MatSym32>), dim3(xcd_blocks_for(g.nn)), dim3(CISM_BLOCK), 0,
-                           c->stream, g,
-                           MatSym32{c->A32}, c->av, c->z32, c->Az32, c->r32, c->partials);
+                           c->stream, g, chunk,
+                           MatSym32{c->A32}, c->av, c->z32, c->Az32, c->r32, c->mpart32);
     else if (((which == 0 && c->sym64_on) || which == 6) && c->a64s_valid) {
         if ((which == 0) == CISM_SYM64_XCD)
             hipLaunchKernelGGL((k_matvec_dots<double, 2, MatSym64<true>>), dim3(xcd_blocks_for(g.nn)),
-                               dim3(CISM_BLOCK), 0, c->stream, g, MatSym64<true>{c->A64s}, c->av, c->z, c->Az,
-                               c->r, c->partials);
+                               dim3(CISM_BLOCK), 0, c->stream, g, chunk, MatSym64<true>{c->A64s}, c->av, c->z,
+                               c->Az, c->r, c->mpart);
         else
             hipLaunchKernelGGL((k_matvec_dots<double, 2, MatSym64<false>>), dim3(nb), dim3(CISM_BLOCK), 0,
-                               c->stream, g, MatSym64<false>{c->A64s}, c->av, c->z, c->Az, c->r, c->partials);
+                               c->stream, g, chunk, MatSym64<false>{c->A64s}, c->av, c->z, c->Az, c->r, c->mpart);
     } else
         hipLaunchKernelGGL((k_matvec_dots<double, 2, MatFull<double>>), dim3(nb), dim3(CISM_BLOCK), 0,
-                           c->stream, g, MatFull<double>{c->A}, c->av, c->z, c->Az, c->r, c->partials);
+                           c->stream, g, chunk, MatFull<double>{c->A}, c->av, c->z, c->Az, c->r, c->mpart);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
 }
