@@ -260,8 +260,10 @@ extern "C" int cism_ctx_create(int nx, int ny, int nz, int nhalo, int periodic, 
         (st = dalloc(&c->as_av_prev, ncol)) || (st = dalloc(&c->as_ac_prev, (size_t)nx * ny)))
         return fail(st);
     if ((st = dalloc(&c->sc, 1))) return fail(st);
-    if (hipHostMalloc(&c->sc_host, sizeof(DevScal), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(&c->sc_host, sizeof(DevScal), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(&c->check, sizeof(CgCheck), hipHostMallocCoherent) != hipSuccess)
         return fail(CISM_ERR_HIP);
+    memset(c->check, 0, sizeof(CgCheck));
     c->a64_valid = 1;
     c->sym64_on = 1;
     *out = c;
@@ -285,6 +287,7 @@ extern "C" int cism_ctx_destroy(cism_ctx *c) {
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (c->sc_host) (void)hipHostFree(c->sc_host);
+    if (c->check) (void)hipHostFree(c->check);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     free(c);
     return CISM_OK;

@@ -48,14 +48,28 @@ struct GridDev {
     long long ne, nepad;      // elements (nz-1)*nx*ny, padded
 };
 
-// device-resident scalars of the CG iterations (one per context)
+// scalars of one CG iteration
+struct CgState {
+    double rho_old, alpha, beta, sigma, eta0, eta1;
+    int nan;   // alpha (or eta1) has been NaN
+};
+
+// device-resident scalars (one per context).  cg: the kernel that uses an iteration's dot
+// products forms its scalars from cg[cur], every workgroup for itself, and workgroup 0
+// leaves them in cg[cur ^ 1] for the next one.
 struct DevScal {
-    double rho_old, alpha, beta, sigma, eta0, eta1, eta2;
-    double L2_rhs, err;
+    CgState cg[2];
+    double L2_rhs;
     double sums[8];
     int nan_flag, singular_flag;
-    int zero_stop;   // inner solves: an exactly zero residual ends the iteration (alpha = 0)
     int beta_bad;    // calcbeta met a negative or NaN beta
+};
+
+// what a convergence check leaves in pinned host memory; seq, the check's number, last
+struct CgCheck {
+    double err;
+    int nan;
+    unsigned seq;
 };
 
 struct cism_guess;   // the learned initial guess of a context (surrogate.hip)
@@ -162,6 +176,8 @@ struct cism_ctx {
     double *red_groups;   // the first pass of a two-pass reduction (RED_GROUPS x CISM_MAX_NV)
     DevScal *sc;
     DevScal *sc_host;   // pinned mirror
+    CgCheck *check;     // pinned, written by the device
+    unsigned check_seq; // number of the last check launched
     // staging for layout conversion (27*nn doubles, lazily)
     double *stage;
     // learned initial guess (cism_learned_guess_load), or null
@@ -399,11 +415,8 @@ void cism_set_error(const char *fmt, ...);
 enum ReduceMode {
     RED_SUMS = 0,       // just the sums
     RED_BB,             // L2_rhs = sqrt(s0)
-    RED_STD_ETA1,       // eta1 = s0; NaN check; beta = eta1/eta0
-    RED_STD_ETA2,       // eta2 = s0; eta0 = eta1; alpha = eta1/eta2; NaN check
-    RED_CG_FIRST,       // rho_old = s0; sigma = s1; alpha = rho_old/sigma
-    RED_CG_ITER,        // Chron-Gear scalars (pcg:1501-1512)
-    RED_ERR,            // err = sqrt(s0)/L2_rhs
+    RED_STD_ETA1,       // eta1 = s0; NaN check; beta = eta1/eta0   (into cg[0])
+    RED_STD_ETA2,       // eta0 = eta1; alpha = eta1/s0; NaN check
     RED_MAX             // max instead of sum (sums[c] = max)
 };
 // part = null: of c->partials

@@ -9,6 +9,7 @@
 #include "internal.h"
 #include "refine_policy.h"
 
+#include <chrono>
 #include <math.h>
 #include <type_traits>
 #include <stdio.h>
@@ -18,49 +19,21 @@
 // ---------------------------------------------------------------------------
 // The scalar step that follows a reduction (mode), on sc->sums.
 __device__ inline void scalar_update(int mode, DevScal *__restrict__ sc) {
-    const double s0 = sc->sums[0], s1 = sc->sums[1];
+    const double s0 = sc->sums[0];
+    CgState &st = sc->cg[0];
     switch (mode) {
     case RED_BB:
         sc->L2_rhs = sqrt(s0);
         break;
     case RED_STD_ETA1:
-        sc->eta1 = s0;
-        if (s0 != s0) sc->nan_flag = 1;
-        sc->beta = sc->eta1 / sc->eta0;
+        st.eta1 = s0;
+        if (s0 != s0) st.nan = 1;
+        st.beta = st.eta1 / st.eta0;
         break;
     case RED_STD_ETA2:
-        sc->eta2 = s0;
-        sc->eta0 = sc->eta1;
-        sc->alpha = sc->eta1 / sc->eta2;
-        if (sc->alpha != sc->alpha) sc->nan_flag = 1;
-        break;
-    case RED_CG_FIRST:
-        sc->rho_old = s0;
-        sc->sigma = s1;
-        if (sc->zero_stop && s0 == 0.0) {
-            sc->alpha = 0.0;
-            break;
-        }
-        sc->alpha = sc->rho_old / sc->sigma;
-        if (sc->alpha != sc->alpha) sc->nan_flag = 1;
-        break;
-    case RED_CG_ITER: {
-        const double rho = s0, delta = s1;
-        if (sc->zero_stop && (rho == 0.0 || sc->rho_old == 0.0)) {
-            sc->alpha = 0.0;
-            sc->beta = 0.0;
-            sc->rho_old = rho;
-            break;
-        }
-        sc->beta = rho / sc->rho_old;
-        sc->sigma = delta - sc->beta * rho / sc->alpha;
-        sc->alpha = rho / sc->sigma;
-        sc->rho_old = rho;
-        if (sc->alpha != sc->alpha) sc->nan_flag = 1;
-        break;
-    }
-    case RED_ERR:
-        sc->err = sqrt(s0) / sc->L2_rhs;
+        st.eta0 = st.eta1;
+        st.alpha = st.eta1 / s0;
+        if (st.alpha != st.alpha) st.nan = 1;
         break;
     default:
         break;
@@ -157,11 +130,152 @@ __global__ void k_reduce_final(const double *__restrict__ groups, int mode, DevS
     if (threadIdx.x == 0) scalar_update(mode, sc);
 }
 
+// The sums of n records of NV partials, formed by the kernel that uses them instead of by two
+// launches before it: every workgroup adds them for itself, in the order of k_reduce_groups
+// (RED_GROUPS groups of `chunk` consecutive records, each by a tree) and k_reduce_final (the
+// groups in turn), so the sums are those two kernels' bit for bit.  chunk <= RED_CHUNK: a
+// lane adds a whole group.  More records go through k_reduce_groups first; its group sums
+// are then 64 records with chunk 1.  With nz = 1, 124 x 136 columns (66 records) the two
+// launches took 2.7 + 4.1 us and two launch gaps of every iteration's 25 us; here the sums
+// take about 1 us of the update kernel.  The line lies at 512 records: each workgroup reads
+// them all from L2, 8 KB, which 2,000 workgroups still do in the time of one launch.
+#define RED_CHUNK 8
+struct RedSrc {
+    const double *p;
+    int n, chunk;
+};
+
+// The sums reach thread 0 only (after the barrier): 64 dependent additions by every lane
+// would cost a full CU more than the launches they replace.
+template <int NV>
+__device__ __forceinline__ void red_sums(const RedSrc &src, double (&out)[NV]) {
+    __shared__ double grp[RED_GROUPS][NV];
+    for (int t = threadIdx.x; t < RED_GROUPS * NV; t += blockDim.x) {
+        const int c = t % NV, b0 = (t / NV) * src.chunk;
+        double v[RED_CHUNK];
+#pragma unroll
+        for (int u = 0; u < RED_CHUNK; ++u)
+            v[u] = u < src.chunk && b0 + u < src.n ? src.p[(size_t)(b0 + u) * NV + c] : 0.0;
+#pragma unroll
+        for (int off = RED_CHUNK / 2; off > 0; off >>= 1)
+#pragma unroll
+            for (int u = 0; u < off; ++u) v[u] += v[u + off];
+        grp[t / NV][c] = v[0];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < NV; ++c) out[c] = grp[0][c];
+#pragma unroll
+        for (int g = 1; g < RED_GROUPS; ++g)
+#pragma unroll
+            for (int c = 0; c < NV; ++c) out[c] += grp[g][c];
+    }
+}
+
 template <int NV>
 static void launch_reduce2(cism_ctx *c, int nb, int mode, const double *part, double *out = nullptr) {
     hipLaunchKernelGGL(k_reduce_groups<NV>, dim3(RED_GROUPS), dim3(CISM_BLOCK), 0, c->stream, part, nb, mode,
                        c->red_groups);
     hipLaunchKernelGGL(k_reduce_final<NV>, dim3(1), dim3(64), 0, c->stream, c->red_groups, mode, c->sc, out);
+}
+
+// the records a consuming kernel adds itself (red_sums)
+template <int NV>
+static RedSrc red_source(cism_ctx *c, const double *part, int nb) {
+    if (nb <= RED_GROUPS * RED_CHUNK) return {part, nb, (nb + RED_GROUPS - 1) / RED_GROUPS};
+    hipLaunchKernelGGL(k_reduce_groups<NV>, dim3(RED_GROUPS), dim3(CISM_BLOCK), 0, c->stream, part, nb,
+                       (int)RED_SUMS, c->red_groups);
+    return {c->red_groups, RED_GROUPS, 1};
+}
+
+// the dot products of a Chron-Gear matvec for the update that follows (of nblk workgroups)
+static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop);
+
+// Chron-Gear's scalars from rho = s0 and delta = s1 (pcg:1390-1405, 1501-1512).  zero_stop
+// (inner solves): an exactly zero residual ends the iteration (alpha = 0).
+__device__ inline CgState cg_step(CgState st, double s0, double s1, int first, int zero_stop) {
+    if (first) {
+        st.rho_old = s0;
+        st.sigma = s1;
+        if (zero_stop && s0 == 0.0) {
+            st.alpha = 0.0;
+            return st;
+        }
+        st.alpha = st.rho_old / st.sigma;
+    } else {
+        if (zero_stop && (s0 == 0.0 || st.rho_old == 0.0)) {
+            st.alpha = 0.0;
+            st.beta = 0.0;
+            st.rho_old = s0;
+            return st;
+        }
+        st.beta = s0 / st.rho_old;
+        st.sigma = s1 - st.beta * s0 / st.alpha;
+        st.alpha = s0 / st.sigma;
+        st.rho_old = s0;
+    }
+    if (st.alpha != st.alpha) st.nan = 1;
+    return st;
+}
+
+// the scalars of a Chron-Gear update: from the dot products' records, or, with no record, as
+// k_cg_scalars left them
+__device__ __forceinline__ void cg_scalars(const RedSrc &src, DevScal *__restrict__ sc, int cur, int first,
+                                           int zero_stop, double &alpha, double &beta) {
+    if (src.n == 0) {
+        alpha = sc->cg[cur ^ 1].alpha;
+        beta = sc->cg[cur ^ 1].beta;
+        return;
+    }
+    __shared__ double ab[2];
+    double dots[2];
+    red_sums<2>(src, dots);
+    if (threadIdx.x == 0) {
+        const CgState st = cg_step(sc->cg[cur], dots[0], dots[1], first, zero_stop);
+        ab[0] = st.alpha;
+        ab[1] = st.beta;
+        if (blockIdx.x == 0) sc->cg[cur ^ 1] = st;
+    }
+    __syncthreads();
+    alpha = ab[0];
+    beta = ab[1];
+}
+
+__global__ __launch_bounds__(CISM_BLOCK) void k_cg_scalars(RedSrc src, DevScal *__restrict__ sc, int cur, int first,
+                                                           int zero_stop) {
+    double alpha, beta;
+    cg_scalars(src, sc, cur, first, zero_stop, alpha, beta);
+}
+
+// one workgroup: |r| / |b| from the partials of (r, r), straight into pinned host memory
+__global__ __launch_bounds__(CISM_BLOCK) void k_cg_check(RedSrc src, const DevScal *__restrict__ sc, int cur,
+                                                         unsigned seq, CgCheck *check) {
+    double s[1];
+    red_sums<1>(src, s);
+    if (threadIdx.x == 0) {
+        check->err = sqrt(s[0]) / sc->L2_rhs;
+        check->nan = sc->cg[cur].nan;
+        __hip_atomic_store(&check->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+// waits until check number c->check_seq has arrived: by reading its number for the first
+// milliseconds (a stream synchronization adds a marker packet and its wake-up, about 8 us of
+// the 60 a small grid's five iterations take), then by synchronizing the stream
+static int cg_check_wait(cism_ctx *c) {
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(&c->check->seq, __ATOMIC_ACQUIRE) != c->check_seq) {
+        for (int i = 0; i < 64; ++i) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            if (__atomic_load_n(&c->check->seq, __ATOMIC_ACQUIRE) != c->check_seq) {
+                cism_set_error("PCG solver: a convergence check did not arrive");
+                return CISM_ERR_HIP;
+            }
+        }
+    }
+    return CISM_OK;
 }
 
 // sums of NV values per block of the partials into out[0..NV), nothing else
@@ -817,7 +931,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_d(long long n2, const T *__r
                                                       const DevScal *__restrict__ sc) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n2) return;
-    const T beta = (T)sc->beta;
+    const T beta = (T)sc->cg[0].beta;
     d[t] = z[t] + beta * d[t];
 }
 
@@ -829,7 +943,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_xr(long long n2, const T *__
                                                        const DevScal *__restrict__ sc) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n2) return;
-    const T alpha = (T)sc->alpha;
+    const T alpha = (T)sc->cg[0].alpha;
     x[t] = x[t] + alpha * d[t];
     r[t] = r[t] - alpha * qv[t];
 }
@@ -898,16 +1012,19 @@ template <typename T>
 __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update(GridDev g, const T *__restrict__ z,
                                                           const T *__restrict__ Az,
                                                           T *__restrict__ d, T *__restrict__ qv,
-                                                          T *__restrict__ x, T *__restrict__ r,
-                                                          const DevScal *__restrict__ sc, int first,
+                                                          T *__restrict__ x, T *__restrict__ r, RedSrc src,
+                                                          DevScal *__restrict__ sc, int cur, int first,
+                                                          int zero_stop,
                                                           const int32_t *__restrict__ skip_av) {
+    double alpha, beta;
+    cg_scalars(src, sc, cur, first, zero_stop, alpha, beta);
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
     const int k = (int)(q % g.nz);
     const long long col = q / g.nz;
     const int i = (int)(col % g.sx), j = (int)(col / g.sx);
     typename Vec2<T>::t rr;
-    cg_update_node<T>(g, q, k, col, i, j, z, Az, d, qv, x, r, (T)sc->alpha, (T)sc->beta, first, skip_av, rr);
+    cg_update_node<T>(g, q, k, col, i, j, z, Az, d, qv, x, r, (T)alpha, (T)beta, first, skip_av, rr);
 }
 
 // The Chron-Gear update followed by the SIA preconditioner of the next iteration
@@ -923,9 +1040,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update(GridDev g, const T *__
 template <typename T, int NZMAX>
 __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T *__restrict__ Az,
                                                        T *__restrict__ d, T *__restrict__ qv,
-                                                       T *__restrict__ x, T *__restrict__ r,
-                                                       const DevScal *__restrict__ sc, int first,
-                                                       const int32_t *__restrict__ av,
+                                                       T *__restrict__ x, T *__restrict__ r, RedSrc src,
+                                                       DevScal *__restrict__ sc, int cur, int first,
+                                                       int zero_stop, const int32_t *__restrict__ av,
                                                        const T *__restrict__ F, int want_rr,
                                                        double *__restrict__ partials, T *__restrict__ colsum,
                                                        const int32_t *__restrict__ um,
@@ -944,7 +1061,9 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
     SiaFactors<T, (NZMAX <= 12 ? NZMAX : 1)> f;
     if constexpr (NZMAX <= 12)
         if (solve) sia_factors<T, NZMAX>(nz, ncol, F, col, comp, f);
-    const T alpha = (T)sc->alpha, beta = (T)sc->beta;
+    double alpha64, beta64;
+    cg_scalars(src, sc, cur, first, zero_stop, alpha64, beta64);
+    const T alpha = (T)alpha64, beta = (T)beta64;
     double acc[1] = {0.0};
     // node t of the block: level t % nz of local column t / nz (32-bit: the context
     // limits grids to 2^30 nodes)
@@ -987,12 +1106,10 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
 // ---------------------------------------------------------------------------
 // PCG drivers
 // ---------------------------------------------------------------------------
-__global__ void k_init_scalars(DevScal *sc, int zero_stop) {
-    sc->rho_old = sc->alpha = sc->beta = sc->sigma = sc->eta1 = sc->eta2 = 0.0;
-    sc->eta0 = 1.0;
-    sc->err = 0.0;
-    sc->nan_flag = 0;
-    sc->zero_stop = zero_stop;
+__global__ void k_init_scalars(DevScal *sc) {
+    CgState st = {};
+    st.eta0 = 1.0;
+    sc->cg[0] = st;
 }
 
 int sync_scalars(cism_ctx *c) {
@@ -1021,8 +1138,20 @@ struct CGVecs {
 // blocks of the fused update (one per 64 columns)
 static inline int sia_blocks(const GridDev &g) { return (int)(((long long)g.sx * g.sy + 63) / 64); }
 
+// An update of more workgroups than this takes its scalars from one workgroup launched before
+// it: every workgroup of the update would wait for the records again (515 x 515 columns at
+// nz = 1, 4,145 workgroups: 190 ms a solve against 201; 163 x 163 x 21, 415: 518 against 523)
+#define CG_FUSE_BLOCKS 1024
+static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop) {
+    const RedSrc src = red_source<2>(c, part, nb);
+    if (nblk <= CG_FUSE_BLOCKS) return src;
+    hipLaunchKernelGGL(k_cg_scalars, dim3(1), dim3(CISM_BLOCK), 0, c->stream, src, c->sc, cur, first, zero_stop);
+    return {nullptr, 0, 0};
+}
+
 template <typename T>
-static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, int first, int want_rr = 0) {
+static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, const RedSrc &src, int cur, int first,
+                            int zero_stop, int want_rr = 0) {
     const GridDev &g = c->g;
     if (precond >= 2) {
         // fused with the SIA preconditioner; the caller skips its own precond call
@@ -1033,21 +1162,25 @@ static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, int first, i
         const int32_t *um = cs && c->dirichlet_any ? c->umask : nullptr;
         const int32_t *vm = cs && c->dirichlet_any ? c->vmask : nullptr;
         if (g.nz <= 12)
-            hipLaunchKernelGGL((k_cg_update_sia<T, 12>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d,
-                               v.q, v.x, v.r, c->sc, first, c->av, v.F, want_rr, c->partials, cs, um, vm);
+            hipLaunchKernelGGL((k_cg_update_sia<T, 12>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
+                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
+                               um, vm);
         else if (g.nz <= 24)
-            hipLaunchKernelGGL((k_cg_update_sia<T, 24>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d,
-                               v.q, v.x, v.r, c->sc, first, c->av, v.F, want_rr, c->partials, cs, um, vm);
+            hipLaunchKernelGGL((k_cg_update_sia<T, 24>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
+                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
+                               um, vm);
         else
-            hipLaunchKernelGGL((k_cg_update_sia<T, 48>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d,
-                               v.q, v.x, v.r, c->sc, first, c->av, v.F, want_rr, c->partials, cs, um, vm);
+            hipLaunchKernelGGL((k_cg_update_sia<T, 48>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
+                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
+                               um, vm);
         HIP_TRY(hipGetLastError());
         if constexpr (std::is_same<T, float>::value)
             if (precond == PRECOND_SIA_COARSE) CISM_TRY(coarse_apply(c, v.z));
         return CISM_OK;
     } else {
         hipLaunchKernelGGL(k_cg_update<T>, dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0, c->stream, g, v.z,
-                           v.Az, v.d, v.q, v.x, v.r, c->sc, first, precond != 0 ? c->av : nullptr);
+                           v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur, first, zero_stop,
+                           precond != 0 ? c->av : nullptr);
     }
     HIP_TRY(hipGetLastError());
     return CISM_OK;
@@ -1070,7 +1203,11 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     const long long np = g.npad;
     // an inner solve (check = 1) whose residual becomes exactly zero has converged; the
     // reference recurrences would divide 0 by 0 there
-    hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, c->stream, c->sc, check);
+    const int zero_stop = check;
+    const int nbu = precond >= 2 ? sia_blocks(g) : nbm;   // workgroups of the update
+    int cur = 0;                // the CgState that holds the current scalars
+    bool checked = false;       // the last launch was a convergence check
+    hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, c->stream, c->sc);
     if (precond == PRECOND_SIA_COARSE && !std::is_same<M, MatSym32>::value) {
         cism_set_error("the coarse correction is a preconditioner of the FP32 inner solves only");
         return CISM_ERR_ARG;
@@ -1098,24 +1235,29 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     auto check_conv = [&](int n, bool &done) -> int {
         // the true residual every fifth iteration, up to the synchronization that reads it
         TimerRange r_c("pcg_matmult_resid", c->stream, true);
+        RedSrc src;
         if (check == 0) {
             hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A,
                                c->av, v.x, v.b, v.r, chrongear, c->partials);
-            CISM_TRY(launch_reduce(c, nbm, 1, RED_ERR));
+            src = red_source<1>(c, c->partials, nbm);
         } else if (chrongear && precond >= 2) {
             // (r, r) came with the fused update of this iteration
-            CISM_TRY(launch_reduce(c, sia_blocks(g), 1, RED_ERR));
+            src = red_source<1>(c, c->partials, sia_blocks(g));
         } else {
             hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, v.r, v.r,
                                c->partials);
-            CISM_TRY(launch_reduce(c, nb, 1, RED_ERR));
+            src = red_source<1>(c, c->partials, nb);
         }
-        CISM_TRY(sync_scalars(c));
-        if (c->sc_host->nan_flag) {
+        hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(CISM_BLOCK), 0, c->stream, src, c->sc, cur,
+                           ++c->check_seq, c->check);
+        HIP_TRY(hipGetLastError());
+        CISM_TRY(cg_check_wait(c));
+        if (c->check->nan) {
             cism_set_error("PCG solver has failed, alpha = NaN");
             return CISM_ERR_NAN;
         }
-        err = c->sc_host->err;
+        checked = true;
+        err = c->check->err;
         done = err < tol;
         if (done) niters = n;
         return CISM_OK;
@@ -1139,6 +1281,7 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
             CISM_TRY(launch_reduce(c, nbr, 1, RED_STD_ETA2, mpart));
             hipLaunchKernelGGL(k_std_xr<T>, dim3(nb2), dim3(CISM_BLOCK), 0, c->stream, 2 * g.nn, v.d,
                                v.q, v.x, v.r, c->sc);
+            checked = false;
             if (n % 5 == 0) {
                 if (check == 0) CISM_TRY((launch_halo_t<T, false>(c, v.x)));
                 CISM_TRY(check_conv(n, done));
@@ -1155,22 +1298,26 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
         CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
         hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk,
                            A, c->av, v.z, v.Az, v.r, mpart);
-        CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_FIRST, mpart));
         // with the SIA preconditioner the update also forms the next z
-        CISM_TRY(launch_cg_update<T>(c, precond, v, 1));
+        CISM_TRY(launch_cg_update<T>(c, precond, v, cg_source(c, mpart, nbr, nbu, cur, 1, zero_stop), cur, 1, zero_stop));
+        cur ^= 1;
         for (int n = 2; n <= maxiters && !done; ++n) {
             if (precond < 2) CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
             hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream,
                                g, chunk, A, c->av, v.z, v.Az, v.r, mpart);
-            CISM_TRY(launch_reduce(c, nbr, 2, RED_CG_ITER, mpart));
-            CISM_TRY(launch_cg_update<T>(c, precond, v, 0, check == 1 && n % 5 == 0));
+            CISM_TRY(launch_cg_update<T>(c, precond, v, cg_source(c, mpart, nbr, nbu, cur, 0, zero_stop), cur, 0, zero_stop,
+                                         check == 1 && n % 5 == 0));
+            cur ^= 1;
+            checked = false;
             if (n % 5 == 0) CISM_TRY(check_conv(n, done));
         }
     }
-    CISM_TRY(sync_scalars(c));
-    if (c->sc_host->nan_flag) {
-        cism_set_error("PCG solver has failed, alpha = NaN");
-        return CISM_ERR_NAN;
+    if (!checked) {
+        CISM_TRY(sync_scalars(c));
+        if (c->sc_host->cg[cur].nan) {
+            cism_set_error("PCG solver has failed, alpha = NaN");
+            return CISM_ERR_NAN;
+        }
     }
     *err_out = err;
     *niters_out = niters;
@@ -1679,7 +1826,8 @@ int launch_cg_matvec(cism_ctx *c, int which) {
 // inner solves issue it (vectors, factors and scalars of the last mixed solve)
 int launch_cg_update32(cism_ctx *c) {
     CGVecs<float> v = {c->x32, c->b32, c->r32, c->d32, c->z32, c->q32, c->Az32, c->F32, nullptr};
-    return launch_cg_update<float>(c, 2, v, 0, 1);
+    const RedSrc src = {c->red_groups, RED_GROUPS, 1};
+    return launch_cg_update<float>(c, 2, v, src, 0, 0, 1, 1);
 }
 
 // sums[0] = |x - xref|^2, sums[1] = |xref|^2 over owned nodes
