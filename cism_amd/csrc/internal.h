@@ -415,8 +415,6 @@ void cism_set_error(const char *fmt, ...);
 enum ReduceMode {
     RED_SUMS = 0,       // just the sums
     RED_BB,             // L2_rhs = sqrt(s0)
-    RED_STD_ETA1,       // eta1 = s0; NaN check; beta = eta1/eta0   (into cg[0])
-    RED_STD_ETA2,       // eta0 = eta1; alpha = eta1/s0; NaN check
     RED_MAX             // max instead of sum (sums[c] = max)
 };
 // part = null: of c->partials

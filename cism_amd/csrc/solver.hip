@@ -12,6 +12,7 @@
 #include <chrono>
 #include <math.h>
 #include <type_traits>
+#include <utility>
 #include <stdio.h>
 
 // ---------------------------------------------------------------------------
@@ -19,25 +20,7 @@
 // ---------------------------------------------------------------------------
 // The scalar step that follows a reduction (mode), on sc->sums.
 __device__ inline void scalar_update(int mode, DevScal *__restrict__ sc) {
-    const double s0 = sc->sums[0];
-    CgState &st = sc->cg[0];
-    switch (mode) {
-    case RED_BB:
-        sc->L2_rhs = sqrt(s0);
-        break;
-    case RED_STD_ETA1:
-        st.eta1 = s0;
-        if (s0 != s0) st.nan = 1;
-        st.beta = st.eta1 / st.eta0;
-        break;
-    case RED_STD_ETA2:
-        st.eta0 = st.eta1;
-        st.alpha = st.eta1 / s0;
-        if (st.alpha != st.alpha) st.nan = 1;
-        break;
-    default:
-        break;
-    }
+    if (mode == RED_BB) sc->L2_rhs = sqrt(sc->sums[0]);
 }
 
 // k_reduce, for any width: one block of 1024 lanes, each with 8 independent
@@ -439,23 +422,18 @@ int launch_matvec64(cism_ctx *c, const double *A, const double *x, double *y) {
     return CISM_OK;
 }
 
-// y = A x plus per-block partial dot products over owned nodes:
-//   NDOT = 1: s0 = (x, y)               [standard PCG (d, Ad)]
-//   NDOT = 2: s0 = (r, x), s1 = (y, x)  [Chron-Gear (r, z), (Az, z)]
-// One lane per node, one pass over the grid; block partials go to a second
-// deterministic pass (k_reduce).
+// y = A x plus per-block partial dot products over owned nodes, s0 = (r, x), s1 = (y, x)
+// (Chron-Gear's (r, z), (Az, z)).  One lane per node, one pass over the grid.
 // FP64, 163 x 163 x 21: 74.2 us with chunks of 128 blocks, 64.1 us with chunks of equal number
 // for every XCD (xcd_chunk_for); 35 x 35 x 10, 46 blocks, 5.9 -> 5.7 us.
-template <typename T, int NDOT, typename M>
+template <typename T, typename M>
 __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, unsigned chunk, const M A,
                                                             const int32_t *__restrict__ av,
                                                             const T *__restrict__ x, T *__restrict__ y,
                                                             const T *__restrict__ r,
                                                             double *__restrict__ partials) {
     using V2 = typename Vec2<T>::t;
-    double acc[NDOT];
-#pragma unroll
-    for (int c = 0; c < NDOT; ++c) acc[c] = 0.0;
+    double acc[2] = {0.0, 0.0};
     const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;
     // a padding block of an XCD grid has no place
     if (M::xcd && lb * blockDim.x >= g.nn) return;
@@ -470,16 +448,12 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, unsigned 
         store2<T>(y, q, yu, yv);
         if (own) {
             const V2 xx = *reinterpret_cast<const V2 *>(x + 2 * q);
-            if (NDOT == 1) {
-                acc[0] = (double)xx.x * (double)yu + (double)xx.y * (double)yv;
-            } else {
-                const V2 rr = *reinterpret_cast<const V2 *>(r + 2 * q);
-                acc[0] = (double)rr.x * (double)xx.x + (double)rr.y * (double)xx.y;
-                acc[NDOT - 1] = (double)yu * (double)xx.x + (double)yv * (double)xx.y;
-            }
+            const V2 rr = *reinterpret_cast<const V2 *>(r + 2 * q);
+            acc[0] = (double)rr.x * (double)xx.x + (double)rr.y * (double)xx.y;
+            acc[1] = (double)yu * (double)xx.x + (double)yv * (double)xx.y;
         }
     }
-    block_reduce_store<NDOT>(acc, partials, M::slots ? xcd_slot(lb) : lb);
+    block_reduce_store<2>(acc, partials, M::slots ? xcd_slot(lb) : lb);
 }
 
 // r = b - A x on the full grid (A x = 0 off owned active rows), s0 = (r, r) over
@@ -924,28 +898,157 @@ int launch_halo_mat(cism_ctx *c, double *A) {
 // ---------------------------------------------------------------------------
 // vector updates (elementwise over the 2*nn interleaved entries)
 // ---------------------------------------------------------------------------
-// standard PCG: d = z + beta*d (pcg:383-393)
-template <typename T>
-__global__ __launch_bounds__(CISM_BLOCK) void k_std_d(long long n2, const T *__restrict__ z,
-                                                      T *__restrict__ d,
-                                                      const DevScal *__restrict__ sc) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n2) return;
-    const T beta = (T)sc->cg[0].beta;
-    d[t] = z[t] + beta * d[t];
+// Standard PCG in two launches an iteration (pcg:300-480).  The direction d = z + beta d
+// and its halo update are formed inside the matvec, which reads z and the old d at a
+// neighbour (at its image for a halo neighbour) and writes the new d to another array: the
+// same operations on the same values as a pass over d, a halo copy and a matvec.  The
+// second launch updates x and r, and with the diagonal or no preconditioner forms the next
+// z and the partials of (r, z) too.  Both form their scalar from the partials they need
+// (red_sums).  35 x 35 x 10, diagonal preconditioner: an iteration was 10 launches of 2.4 to
+// 6 us, 42 us in all (187 ms a solve); two take 12.2 + 4.1 us, 24 us with the checks (105 ms).
+
+// beta = (r, z) / the last (r, z)   (pcg:366-382)
+__device__ inline CgState std_beta_step(CgState st, double s0) {
+    st.eta1 = s0;
+    if (s0 != s0) st.nan = 1;
+    st.beta = st.eta1 / st.eta0;
+    return st;
+}
+// alpha = (r, z) / (d, A d)   (pcg:440-463)
+__device__ inline CgState std_alpha_step(CgState st, double s0) {
+    st.eta0 = st.eta1;
+    st.alpha = st.eta1 / s0;
+    if (st.alpha != st.alpha) st.nan = 1;
+    return st;
 }
 
-// standard PCG: x += alpha*d, r -= alpha*q (pcg:466-472)
-template <typename T>
-__global__ __launch_bounds__(CISM_BLOCK) void k_std_xr(long long n2, const T *__restrict__ d,
-                                                       const T *__restrict__ qv, T *__restrict__ x,
-                                                       T *__restrict__ r,
-                                                       const DevScal *__restrict__ sc) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n2) return;
-    const T alpha = (T)sc->cg[0].alpha;
-    x[t] = x[t] + alpha * d[t];
-    r[t] = r[t] - alpha * qv[t];
+template <typename T, typename M>
+__global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned chunk, const M A,
+                                                           const int32_t *__restrict__ av,
+                                                           const T *__restrict__ z, const T *__restrict__ d,
+                                                           T *__restrict__ dn, T *__restrict__ y, RedSrc src,
+                                                           DevScal *__restrict__ sc, int cur,
+                                                           double *__restrict__ partials) {
+    using V2 = typename Vec2<T>::t;
+    const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;
+    if (M::xcd && lb * blockDim.x >= g.nn) return;
+    __shared__ double sb;
+    {
+        double s[1];
+        red_sums<1>(src, s);
+        if (threadIdx.x == 0) {
+            const CgState st = std_beta_step(sc->cg[cur], s[0]);
+            sb = st.beta;
+            if (blockIdx.x == 0) sc->cg[cur ^ 1] = st;
+        }
+        __syncthreads();
+    }
+    const T beta = (T)sb;
+    double acc[1] = {0.0};
+    const long long q = lb * blockDim.x + threadIdx.x;
+    if (q < g.nn) {
+        const int k = (int)(q % g.nz);
+        const long long col = q / g.nz;
+        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        // the first node of the image of a column, or -1
+        auto image = [&](int ii, int jj) {
+            const int im = halo_image(ii, g.sx, g.periodic), jm = halo_image(jj, g.sy, g.periodic);
+            return im >= 0 && jm >= 0 ? (long long)g.nz * (im + (long long)g.sx * jm) : -1;
+        };
+        // the new d of level kk of an image column (0 without one); every load unconditional
+        auto dir = [&](long long base, int kk) {
+            const long long p = (base >= 0 ? base : 0) + kk;
+            const V2 zz = reinterpret_cast<const V2 *>(z)[p], dd = reinterpret_cast<const V2 *>(d)[p];
+            V2 v;
+            v.x = base >= 0 ? zz.x + beta * dd.x : (T)0;
+            v.y = base >= 0 ? zz.y + beta * dd.y : (T)0;
+            return v;
+        };
+        const V2 own = dir(image(i, j), k);
+        T su = 0, sv = 0;
+        if (is_owned(g, i, j) && av[col]) {
+            long long nb[9];
+#pragma unroll
+            for (int o = 0; o < 9; ++o) nb[o] = image(i + o % 3 - 1, j + o / 3 - 1);
+            // the row product's order and operations (row_product)
+#pragma unroll
+            for (int kA = -1; kA <= 1; ++kA) {
+                if (k + kA < 0 || k + kA >= g.nz) continue;
+#pragma unroll
+                for (int o = 0; o < 9; ++o) {
+                    const int iA = o % 3 - 1, jA = o / 3 - 1;
+                    const V2 xx = dir(nb[o], k + kA);
+                    T uu, uv, vu, vv;
+                    A.blocks(q, slot_of(iA, jA, kA), q + kA + (long long)g.nz * (iA + (long long)g.sx * jA), uu, uv,
+                             vu, vv);
+                    su = su + uu * xx.x + uv * xx.y;
+                    sv = sv + vu * xx.x + vv * xx.y;
+                }
+            }
+        }
+        store2<T>(dn, q, own.x, own.y);
+        store2<T>(y, q, su, sv);
+        if (is_owned(g, i, j)) acc[0] = (double)own.x * (double)su + (double)own.y * (double)sv;
+    }
+    block_reduce_store<1>(acc, partials, lb);
+}
+
+// z = M^-1 r of node q, M the diagonal (precond 1) or nothing (0)
+template <typename T, typename M>
+__device__ __forceinline__ typename Vec2<T>::t point_precond(const GridDev &g, const M &A, int precond,
+                                                             long long q, typename Vec2<T>::t r) {
+    if (precond == 0) return r;
+    const T du = A.entry(g, 0, CISM_DIAG, q), dv = A.entry(g, 3, CISM_DIAG, q);
+    typename Vec2<T>::t z;
+    z.x = du != (T)0 ? r.x / du : (T)0;
+    z.y = dv != (T)0 ? r.y / dv : (T)0;
+    return z;
+}
+
+// x += alpha d, r -= alpha q (pcg:466-472); with precond 0 or 1 also z = M^-1 r and the
+// partials of (r, z), in k_dot's order (its grid).  update = 0: z and (r, z) alone.
+template <typename T, typename M>
+__global__ __launch_bounds__(CISM_BLOCK) void k_std_update(GridDev g, const M A, int precond, int update,
+                                                           const T *__restrict__ d, const T *__restrict__ qv,
+                                                           T *__restrict__ x, T *__restrict__ r, T *__restrict__ z,
+                                                           RedSrc src, DevScal *__restrict__ sc, int cur,
+                                                           double *__restrict__ partials) {
+    using V2 = typename Vec2<T>::t;
+    T alpha = (T)0;
+    if (update) {
+        __shared__ double sa;
+        double s[1];
+        red_sums<1>(src, s);
+        if (threadIdx.x == 0) {
+            const CgState st = std_alpha_step(sc->cg[cur], s[0]);
+            sa = st.alpha;
+            if (blockIdx.x == 0) sc->cg[cur ^ 1] = st;
+        }
+        __syncthreads();
+        alpha = (T)sa;
+    }
+    double acc[1] = {0.0};
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
+        V2 rr = reinterpret_cast<const V2 *>(r)[q];
+        if (update) {
+            const V2 dd = reinterpret_cast<const V2 *>(d)[q], qq = reinterpret_cast<const V2 *>(qv)[q];
+            V2 xx = reinterpret_cast<const V2 *>(x)[q];
+            xx.x = xx.x + alpha * dd.x;
+            xx.y = xx.y + alpha * dd.y;
+            rr.x = rr.x - alpha * qq.x;
+            rr.y = rr.y - alpha * qq.y;
+            reinterpret_cast<V2 *>(x)[q] = xx;
+            reinterpret_cast<V2 *>(r)[q] = rr;
+        }
+        if (precond <= 1) {
+            const V2 zz = point_precond<T>(g, A, precond, q, rr);
+            reinterpret_cast<V2 *>(z)[q] = zz;
+            const int col = (int)(q / g.nz), j = col / g.sx, i = col - j * g.sx;
+            if (is_owned(g, i, j)) acc[0] += (double)rr.x * (double)zz.x + (double)rr.y * (double)zz.y;
+        }
+    }
+    if (precond <= 1) block_reduce_store<1>(acc, partials);
 }
 
 // Chron-Gear (pcg:1517-1536) of node q with the halo update of Az (pcg:1494-1497)
@@ -1268,19 +1371,28 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
         CISM_TRY((launch_halo_t<T, false>(c, v.x)));
         hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
                            v.x, v.b, v.r, 0, c->partials);
+        T *d = v.d, *dn = v.Az;   // the direction and where the next one goes
         for (int n = 1; n <= maxiters && !done; ++n) {
-            CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
-            hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, v.r, v.z,
-                               c->partials);
-            CISM_TRY(launch_reduce(c, nb, 1, RED_STD_ETA1));
-            hipLaunchKernelGGL(k_std_d<T>, dim3(nb2), dim3(CISM_BLOCK), 0, c->stream, 2 * g.nn, v.z,
-                               v.d, c->sc);
-            CISM_TRY((launch_halo_t<T, false>(c, v.d)));
-            hipLaunchKernelGGL((k_matvec_dots<T, 1, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g,
-                               chunk, A, c->av, v.d, v.q, (const T *)nullptr, mpart);
-            CISM_TRY(launch_reduce(c, nbr, 1, RED_STD_ETA2, mpart));
-            hipLaunchKernelGGL(k_std_xr<T>, dim3(nb2), dim3(CISM_BLOCK), 0, c->stream, 2 * g.nn, v.d,
-                               v.q, v.x, v.r, c->sc);
+            // z and (r, z): with a point preconditioner the last update has formed them
+            // unless the check has replaced r since
+            if (precond >= 2) {
+                CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
+                hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, v.r, v.z,
+                                   c->partials);
+            } else if (n % 5 == 1) {
+                hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 0,
+                                   d, v.q, v.x, v.r, v.z, RedSrc{}, c->sc, cur, c->partials);
+            }
+            const RedSrc s1 = red_source<1>(c, c->partials, nb);
+            hipLaunchKernelGGL((k_std_matvec<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
+                               v.z, d, dn, v.q, s1, c->sc, cur, mpart);
+            cur ^= 1;
+            std::swap(d, dn);
+            const RedSrc s2 = red_source<1>(c, mpart, nbr);
+            hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 1, d,
+                               v.q, v.x, v.r, v.z, s2, c->sc, cur, c->partials);
+            cur ^= 1;
+            HIP_TRY(hipGetLastError());
             checked = false;
             if (n % 5 == 0) {
                 if (check == 0) CISM_TRY((launch_halo_t<T, false>(c, v.x)));
@@ -1296,14 +1408,14 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
                                v.x, v.b, v.r, 1, c->partials);
         }
         CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
-        hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk,
+        hipLaunchKernelGGL((k_matvec_dots<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk,
                            A, c->av, v.z, v.Az, v.r, mpart);
         // with the SIA preconditioner the update also forms the next z
         CISM_TRY(launch_cg_update<T>(c, precond, v, cg_source(c, mpart, nbr, nbu, cur, 1, zero_stop), cur, 1, zero_stop));
         cur ^= 1;
         for (int n = 2; n <= maxiters && !done; ++n) {
             if (precond < 2) CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
-            hipLaunchKernelGGL((k_matvec_dots<T, 2, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream,
+            hipLaunchKernelGGL((k_matvec_dots<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream,
                                g, chunk, A, c->av, v.z, v.Az, v.r, mpart);
             CISM_TRY(launch_cg_update<T>(c, precond, v, cg_source(c, mpart, nbr, nbu, cur, 0, zero_stop), cur, 0, zero_stop,
                                          check == 1 && n % 5 == 0));
@@ -1804,19 +1916,19 @@ int launch_cg_matvec(cism_ctx *c, int which) {
     const int nb = nblocks_for(g.nn);
     const unsigned chunk = xcd_chunk_for(g.nn);
     if (which == 1)
-        hipLaunchKernelGGL((k_matvec_dots<float, 2, MatSym32>), dim3(xcd_blocks_for(g.nn)), dim3(CISM_BLOCK), 0,
+        hipLaunchKernelGGL((k_matvec_dots<float, MatSym32>), dim3(xcd_blocks_for(g.nn)), dim3(CISM_BLOCK), 0,
                            c->stream, g, chunk,
                            MatSym32{c->A32}, c->av, c->z32, c->Az32, c->r32, c->mpart32);
     else if (((which == 0 && c->sym64_on) || which == 6) && c->a64s_valid) {
         if ((which == 0) == CISM_SYM64_XCD)
-            hipLaunchKernelGGL((k_matvec_dots<double, 2, MatSym64<true>>), dim3(xcd_blocks_for(g.nn)),
+            hipLaunchKernelGGL((k_matvec_dots<double, MatSym64<true>>), dim3(xcd_blocks_for(g.nn)),
                                dim3(CISM_BLOCK), 0, c->stream, g, chunk, MatSym64<true>{c->A64s}, c->av, c->z,
                                c->Az, c->r, c->mpart);
         else
-            hipLaunchKernelGGL((k_matvec_dots<double, 2, MatSym64<false>>), dim3(nb), dim3(CISM_BLOCK), 0,
+            hipLaunchKernelGGL((k_matvec_dots<double, MatSym64<false>>), dim3(nb), dim3(CISM_BLOCK), 0,
                                c->stream, g, chunk, MatSym64<false>{c->A64s}, c->av, c->z, c->Az, c->r, c->mpart);
     } else
-        hipLaunchKernelGGL((k_matvec_dots<double, 2, MatFull<double>>), dim3(nb), dim3(CISM_BLOCK), 0,
+        hipLaunchKernelGGL((k_matvec_dots<double, MatFull<double>>), dim3(nb), dim3(CISM_BLOCK), 0,
                            c->stream, g, chunk, MatFull<double>{c->A}, c->av, c->z, c->Az, c->r, c->mpart);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
