@@ -45,228 +45,302 @@ __device__ inline short f2bf(float f) {
 // ---------------------------------------------------------------------------
 // implicit-GEMM convolution: out[p][co] = act(bias[co] + sum_k W[co][k] * X(p, k))
 // k = tap*Ci + ci, tap = ky*3 + kx (ks = 3) or 0 (ks = 1); X(p, k) = in at pixel p
-// shifted by (ky-1, kx-1) with periodic wrap.  Requires Ci % 16 == 0.
-// Block tile: 64 output channels x 64 pixels, 4 waves of 2x2 16x16 MFMA tiles.
+// shifted by (ky-1, kx-1) with periodic wrap.  Ci is a multiple of 16, Co of 32.
 // ---------------------------------------------------------------------------
 struct ConvDims {
     int B, H, W, Ci, Co, ks, relu;
 };
 
-__device__ inline long long shifted_pixel(long long p, int tap, int ks, int H, int W) {
-    if (ks == 1) return p;
-    const int HW = H * W;
-    const long long b = p / HW;
-    const int r = (int)(p - b * HW);
-    int y = r / W, x = r - (r / W) * W;
-    y += tap / 3 - 1;
-    x += tap % 3 - 1;
-    y = y < 0 ? y + H : (y >= H ? y - H : y);
-    x = x < 0 ? x + W : (x >= W ? x - W : x);
-    return b * HW + (long long)y * W + x;
+// A convolution's input: one image a of Ca channels, or (b not null) the decoder's
+// concatenation, read in place: channels [0, Ca) from a at half the resolution (nearest
+// upsampling), the Cb after them from b.  Ca and Cb are multiples of 8 (of 32 with b).
+struct ConvSrc {
+    const float *a, *b;
+    int Ca, Cb;
+};
+
+// Images are worked on in patches of 8 x 8 output pixels.
+#define CONV_P 8
+
+// 8 channels from c of pixel (y, x) of image n (y, x inside the image) as BF16
+__device__ __forceinline__ const float *conv_src_at(const ConvDims &d, const ConvSrc &s, int n, int y, int x, int c) {
+    if (!s.b) return s.a + (((long long)n * d.H + y) * d.W + x) * s.Ca + c;
+    if (c < s.Ca) return s.a + (((long long)n * (d.H >> 1) + (y >> 1)) * (d.W >> 1) + (x >> 1)) * s.Ca + c;
+    return s.b + (((long long)n * d.H + y) * d.W + x) * s.Cb + (c - s.Ca);
 }
 
-// K values staged in LDS per step of the forward convolution: 2 MFMA k-steps of 32
-// between two barriers; a thread stages 16 consecutive k of one weight row and of one
-// pixel (Ci % 16 == 0, so the 16 lie in one tap and their 3x3 shift is computed once).
-// A K that is not a multiple of 32 (3x3 over 16 channels: 144) ends in staged zeros.
+__device__ __forceinline__ uint4 pack_bf16(const float4 &f, const float4 &h) {
+    auto two = [](float lo, float hi) {
+        return (unsigned)(unsigned short)f2bf(lo) | ((unsigned)(unsigned short)f2bf(hi) << 16);
+    };
+    return make_uint4(two(f.x, f.y), two(f.z, f.w), two(h.x, h.y), two(h.z, h.w));
+}
+
+// source of patch pixel (ly, lx) of a patch with a halo of `off` pixels whose first output
+// pixel is (y0, x0): the wrapped coordinates, or false for a pixel no output needs
+__device__ __forceinline__ bool patch_pixel(const ConvDims &d, int off, int y0, int x0, int ly, int lx, int &y,
+                                            int &x) {
+    y = y0 + ly - off;
+    x = x0 + lx - off;
+    if (y >= d.H + off || x >= d.W + off) return false;
+    y = y < 0 ? y + d.H : (y >= d.H ? y - d.H : y);
+    x = x < 0 ? x + d.W : (x >= d.W ? x - d.W : x);
+    return true;
+}
+
+// One workgroup: 32 NA output channels of one patch; wave (w >> 1, w & 1) takes 16 NA of the
+// channels and 32 of the pixels (4 patch rows), NA x 2 MFMA tiles.  The patch with its halo is
+// staged once, as BF16, all Ci channels of a pixel together: each input value is loaded and
+// converted once per workgroup instead of once per tap, and every tap's operand is the same
+// rows of LDS at another pixel offset.  The row stride Ci + 8 puts the 16-byte reads of eight
+// neighbouring pixels on disjoint banks for every Ci here.  The weights come from L2 in the
+// order the MFMA reads them (Wf[co / 16][k / 32][lane][8], k_prep_weights): 1 KB contiguous
+// per fragment.  k ascends in steps of 32 from one accumulator, zeros past K (3x3 over 16
+// channels: 144), so an output does not depend on the tiling.
 // Lane l of an MFMA holds row (l & 15) of A and column (l & 15) of B with 8 consecutive
 // k from 8 (l >> 4); its 4 results are rows 4 (l >> 4) + i of column (l & 15).
-#define CONV_CK 64
-
-__global__ __launch_bounds__(256) void k_conv_mfma(ConvDims d, const float *__restrict__ in,
-                                                   const short *__restrict__ Wb,
-                                                   const float *__restrict__ bias,
-                                                   float *__restrict__ out) {
-    alignas(16) __shared__ short As[64][CONV_CK + 8];   // weights [co][k]
-    alignas(16) __shared__ short Bs[64][CONV_CK + 8];   // inputs [pixel][k]
-    const int K = d.ks * d.ks * d.Ci;
-    const int HW = d.H * d.W;
-    const long long P = (long long)d.B * HW;
-    const int co0 = blockIdx.y * 64;
-    const long long p0 = (long long)blockIdx.x * 64;
+// mask (the data gradient of an input that went through a ReLU): zero where mask is not
+// positive.
+// Bound: the MFMA operands' L1 and LDS reads (2 + 2 KB per 4 MFMAs of a wave) at the deep
+// levels, the FP32 activations' traffic at the full resolution.  The twelve layers at 512 x 512:
+// 0.64 ms with every tap loaded and converted again and the concatenations written out,
+// 0.27 ms here.
+template <int NA>
+__global__ __launch_bounds__(256) void k_conv_patch(ConvDims d, ConvSrc src, const short *__restrict__ Wf,
+                                                    const float *__restrict__ bias, const float *__restrict__ mask,
+                                                    float *__restrict__ out) {
+    extern __shared__ __align__(16) short X[];   // [pixel][Ci + 8]
+    const int ld = d.Ci + 8, off = d.ks == 3 ? 1 : 0, R = CONV_P + 2 * off, G = d.Ci >> 3;
+    const int tw = (d.W + CONV_P - 1) / CONV_P, th = (d.H + CONV_P - 1) / CONV_P;
+    const int n = blockIdx.x / (tw * th), pt = blockIdx.x - n * (tw * th);
+    const int y0 = pt / tw * CONV_P, x0 = (pt - pt / tw * tw) * CONV_P;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wc = (wave >> 1) * 32, wp = (wave & 1) * 32;
-    f32x4 acc[2][2];
-    for (int a = 0; a < 2; ++a)
+    const int items = R * R * G;   // 8 channels of a pixel each
+    for (int i0 = t; i0 < items; i0 += 4 * 256) {
+        float4 v[4][2];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int it = i0 + u * 256, px = it / G, ly = px / R;
+            int y, x;
+            v[u][0] = v[u][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (it < items && patch_pixel(d, off, y0, x0, ly, px - ly * R, y, x)) {
+                const float4 *p = reinterpret_cast<const float4 *>(conv_src_at(d, src, n, y, x, (it - px * G) * 8));
+                v[u][0] = p[0];
+                v[u][1] = p[1];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int it = i0 + u * 256, px = it / G;
+            if (it < items) *reinterpret_cast<uint4 *>(&X[px * ld + (it - px * G) * 8]) = pack_bf16(v[u][0], v[u][1]);
+        }
+    }
+    __syncthreads();
+    const int K = d.ks * d.ks * d.Ci, S = (K + 31) >> 5;
+    const int co0 = blockIdx.y * 32 * NA + (wave >> 1) * 16 * NA, row0 = (wave & 1) * 4;
+    f32x4 acc[NA][2];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const int lr = t >> 2, lk = (t & 3) * 16;   // loader: row / pixel lr, 16 k values from lk
-    const int co = co0 + lr;
-    const long long p = p0 + lr;
-    const bool pok = p < P, cok = co < d.Co;
-    // the loader pixel's image coordinates, once
-    long long pb = 0;
-    int py = 0, px = 0;
-    if (pok) {
-        pb = p / HW;
-        const int r = (int)(p - pb * HW);
-        py = r / d.W;
-        px = r - py * d.W;
+    const bf16x8 *wf = reinterpret_cast<const bf16x8 *>(Wf) + (long long)(co0 >> 4) * S * 64 + lane;
+    // this lane's pixel of the two B tiles, and its k within the step as (tap, channel)
+    const int c15 = lane & 15;
+    const short *xb0 = X + ((row0 + (c15 >> 3)) * R + (c15 & 7)) * ld;
+    const short *xb1 = xb0 + 2 * R * ld;
+    int tap = 0, ci = 8 * (lane >> 4);
+    if (ci >= d.Ci) {   // Ci = 16: the step's second half is the next tap
+        ci -= d.Ci;
+        tap = 1;
     }
-    for (int k0 = 0; k0 < K; k0 += CONV_CK) {
-        const int k = k0 + lk;
-        uint4 a0 = {0u, 0u, 0u, 0u}, a1 = {0u, 0u, 0u, 0u};
-        if (cok && k < K) {
-            const uint4 *src = reinterpret_cast<const uint4 *>(Wb + (long long)co * K + k);
-            a0 = src[0];
-            a1 = src[1];
-        }
-        *reinterpret_cast<uint4 *>(&As[lr][lk]) = a0;
-        *reinterpret_cast<uint4 *>(&As[lr][lk + 8]) = a1;
-        if (pok && k < K) {
-            const int tap = k / d.Ci, ci = k - tap * d.Ci;
-            long long src = p;
-            if (d.ks == 3) {
-                int y = py + tap / 3 - 1, x = px + tap % 3 - 1;
-                y = y < 0 ? y + d.H : (y >= d.H ? y - d.H : y);
-                x = x < 0 ? x + d.W : (x >= d.W ? x - d.W : x);
-                src = pb * HW + (long long)y * d.W + x;
-            }
-            // 16 BF16 values packed two per word: two 16-byte LDS stores
-            const float4 *v = reinterpret_cast<const float4 *>(in + src * d.Ci + ci);
-            unsigned w[8];
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+        bf16x8 af[NA], b0, b1;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 f = v[q];
-                w[2 * q] = (unsigned)(unsigned short)f2bf(f.x) | ((unsigned)(unsigned short)f2bf(f.y) << 16);
-                w[2 * q + 1] = (unsigned)(unsigned short)f2bf(f.z) | ((unsigned)(unsigned short)f2bf(f.w) << 16);
-            }
-            *reinterpret_cast<uint4 *>(&Bs[lr][lk]) = make_uint4(w[0], w[1], w[2], w[3]);
-            *reinterpret_cast<uint4 *>(&Bs[lr][lk + 8]) = make_uint4(w[4], w[5], w[6], w[7]);
+        for (int a = 0; a < NA; ++a) af[a] = wf[((long long)a * S + s) * 64];
+        const int ky = tap / 3, o = (ky * R + tap - 3 * ky) * ld + ci;
+        if (tap < d.ks * d.ks) {
+            b0 = *reinterpret_cast<const bf16x8 *>(xb0 + o);
+            b1 = *reinterpret_cast<const bf16x8 *>(xb1 + o);
         } else {
-            *reinterpret_cast<uint4 *>(&Bs[lr][lk]) = make_uint4(0u, 0u, 0u, 0u);
-            *reinterpret_cast<uint4 *>(&Bs[lr][lk + 8]) = make_uint4(0u, 0u, 0u, 0u);
+            b0 = b1 = bf16x8{};
         }
-        __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < CONV_CK; kk += 32) {
-            if (k0 + kk >= K) break;   // the same for the whole block
-            bf16x8 af[2], bfm[2];
-            for (int a = 0; a < 2; ++a) {
-                const int row = wc + a * 16 + (lane & 15);
-                af[a] = *reinterpret_cast<const bf16x8 *>(&As[row][kk + 8 * (lane >> 4)]);
-            }
-            for (int b = 0; b < 2; ++b) {
-                const int col = wp + b * 16 + (lane & 15);
-                bfm[b] = *reinterpret_cast<const bf16x8 *>(&Bs[col][kk + 8 * (lane >> 4)]);
-            }
-            for (int a = 0; a < 2; ++a)
-                for (int b = 0; b < 2; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfm[b], acc[a][b], 0, 0, 0);
+        for (int a = 0; a < NA; ++a) {
+            acc[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], b0, acc[a][0], 0, 0, 0);
+            acc[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], b1, acc[a][1], 0, 0, 0);
         }
-        __syncthreads();
+        ci += 32;
+        while (ci >= d.Ci) {
+            ci -= d.Ci;
+            ++tap;
+        }
     }
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int y = y0 + row0 + 2 * b + (c15 >> 3), x = x0 + (c15 & 7);
+        if (y >= d.H || x >= d.W) continue;
+        const long long p = ((long long)n * d.H + y) * d.W + x;
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            const int oc = co0 + 16 * a + 4 * (lane >> 4);
+            float v[4];
+#pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int oc = co0 + wc + a * 16 + 4 * (lane >> 4) + i;
-                const long long op = p0 + wp + b * 16 + (lane & 15);
-                if (oc < d.Co && op < P) {
-                    float v = acc[a][b][i] + (bias ? bias[oc] : 0.f);
-                    if (d.relu) v = v > 0.f ? v : 0.f;
-                    out[op * d.Co + oc] = v;
-                }
+                v[i] = acc[a][b][i] + (bias ? bias[oc + i] : 0.f);
+                if (d.relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
             }
+            if (mask) {
+                const float4 m = *reinterpret_cast<const float4 *>(mask + p * d.Co + oc);
+                v[0] = m.x > 0.f ? v[0] : 0.f;
+                v[1] = m.y > 0.f ? v[1] : 0.f;
+                v[2] = m.z > 0.f ? v[2] : 0.f;
+                v[3] = m.w > 0.f ? v[3] : 0.f;
+            }
+            *reinterpret_cast<float4 *>(out + p * d.Co + oc) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+    }
 }
 
-// weight gradient: dW[co][k] = sum_p dY[p][co] * X(p, k); pixel range split over
-// gridDim.z, partial tiles reduced by k_wgrad_reduce (fixed order).
-__global__ __launch_bounds__(256) void k_wgrad_mfma(ConvDims d, const float *__restrict__ dY,
-                                                    const float *__restrict__ X,
-                                                    float *__restrict__ part, long long pchunk) {
-    alignas(16) __shared__ short As[64][32 + 8];   // [co][pix]
-    alignas(16) __shared__ short Bs[64][32 + 8];   // [k][pix]
-    const int K = d.ks * d.ks * d.Ci;
-    const long long P = (long long)d.B * d.H * d.W;
-    const int co0 = blockIdx.y * 64, kq0 = blockIdx.x * 64;
-    const long long pbeg = (long long)blockIdx.z * pchunk;
-    const long long pend = pbeg + pchunk < P ? pbeg + pchunk : P;
+// Weight and bias gradients: dW[co][k] = sum_p dY[p][co] * X(p, k), db[co] = sum_p dY[p][co].
+// One workgroup: 32 output x 32 input channels, every tap, over a run of patches; wave
+// (w >> 1, w & 1) has 16 x 16 of them, KS * KS MFMA tiles.  The contraction runs over pixels,
+// which neither operand has contiguous: both patches are staged [pixel][channel] as BF16
+// and gfx950's transposing LDS reads (ds_read_b64_tr_b16: 16 lanes read 4 pixels x 16
+// channels, each lane receives one channel of the 4 pixels) give the MFMA's 8 consecutive
+// pixels of a channel in two reads.  A k step of 32 is 4 patch rows.  dY is staged once for
+// the nine taps, and the next patch is loaded while this one is multiplied.  The bias
+// gradient adds the loader's FP32 values of dY (the workgroups of the first 32 input
+// channels).  Partials per run, part[run][Co * K weights, then Co biases], are added by
+// k_wgrad_reduce in a fixed order.  A patch's staging (FP32 loads and conversions) bounds it
+// at 32 x 32 channels.  The twelve layers at 4 x 256 x 256, with the reductions: 4.9 ms with
+// dY and X staged transposed once per tap and a pass per channel for the biases, 0.35 ms here.
+#define WG_LD 48   // staged channels of a pixel: 32 and a pad that keeps 4 pixels on disjoint banks
+template <int KS>
+__global__ __launch_bounds__(256) void k_wgrad_patch(ConvDims d, ConvSrc src, const float *__restrict__ dY,
+                                                     float *__restrict__ part, int per) {
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    typedef short s8 __attribute__((ext_vector_type(8)));
+    constexpr int OFF = KS == 3 ? 1 : 0, R = CONV_P + 2 * OFF, NX = (R * R * 4 + 255) / 256;
+    alignas(16) __shared__ short Ys[CONV_P * CONV_P * WG_LD];
+    alignas(16) __shared__ short Xs[R * R * WG_LD];
+    const int tw = (d.W + CONV_P - 1) / CONV_P, th = (d.H + CONV_P - 1) / CONV_P, np = d.B * tw * th;
+    const int ci0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
+    const int q0 = blockIdx.z * per, q1 = min(np, q0 + per);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wc = (wave >> 1) * 32, wk = (wave & 1) * 32;
-    f32x4 acc[2][2];
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const int lp = t >> 4, lc = (t & 15) * 4;     // loader: pixels lp and lp + 16, 4 values from lc
-    // the B loader's tap and channel are fixed for the block
-    const int kl = kq0 + lc;
-    const int ltap = kl < K ? kl / d.Ci : 0, lci = kl < K ? kl - ltap * d.Ci : 0;
-    for (long long q0 = pbeg; q0 < pend; q0 += 32) {
+    float4 vy[2], vx[NX][2];
+    float bsum[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) bsum[c] = 0.f;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load = [&](int q) {
+        const int n = q / (tw * th), pt = q - n * (tw * th);
+        const int y0 = pt / tw * CONV_P, x0 = (pt - pt / tw * tw) * CONV_P;
+        {
+            const int y = y0 + (t >> 5), x = x0 + ((t >> 2) & 7);
+            vy[0] = vy[1] = zero;
+            if (y < d.H && x < d.W) {
+                const float4 *p = reinterpret_cast<const float4 *>(
+                    dY + (((long long)n * d.H + y) * d.W + x) * d.Co + co0 + 8 * (t & 3));
+                vy[0] = p[0];
+                vy[1] = p[1];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            const int it = t + 256 * u, px = it >> 2, ly = px / R, c = ci0 + 8 * (it & 3);
+            int y, x;
+            vx[u][0] = vx[u][1] = zero;
+            if (px < R * R && c < d.Ci && patch_pixel(d, OFF, y0, x0, ly, px - ly * R, y, x)) {
+                const float4 *p = reinterpret_cast<const float4 *>(conv_src_at(d, src, n, y, x, c));
+                vx[u][0] = p[0];
+                vx[u][1] = p[1];
+            }
+        }
+    };
+    f32x4 acc[KS * KS];
+#pragma unroll
+    for (int k = 0; k < KS * KS; ++k) acc[k] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int g = lane >> 4, l4 = (lane & 15) >> 2, ch = 4 * (lane & 3);
+    // 8 consecutive pixels of one channel: two transposing reads of 4 pixels
+    auto frag = [&](const short *p) {
+        using lds4 = __attribute__((address_space(3))) s4;
+        const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+        const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 4 * WG_LD));
+        const s8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        return __builtin_bit_cast(bf16x8, v);
+    };
+    if (q0 < q1) load(q0);
+    for (int q = q0; q < q1; ++q) {
+        __syncthreads();   // the last patch's reads are done
+        *reinterpret_cast<uint4 *>(&Ys[(t >> 2) * WG_LD + 8 * (t & 3)]) = pack_bf16(vy[0], vy[1]);
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            const int it = t + 256 * u;
+            if ((it >> 2) < R * R)
+                *reinterpret_cast<uint4 *>(&Xs[(it >> 2) * WG_LD + 8 * (it & 3)]) = pack_bf16(vx[u][0], vx[u][1]);
+        }
+        bsum[0] += vy[0].x; bsum[1] += vy[0].y; bsum[2] += vy[0].z; bsum[3] += vy[0].w;
+        bsum[4] += vy[1].x; bsum[5] += vy[1].y; bsum[6] += vy[1].z; bsum[7] += vy[1].w;
+        __syncthreads();
+        if (q + 1 < q1) load(q + 1);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int pl = lp + 16 * h;
-            const long long p = q0 + pl;
-            const bool okp = p < pend;
-            {   // A: dY[p][co0+lc..+3] -> As[co][pix]
-                float4 v = {0.f, 0.f, 0.f, 0.f};
-                if (okp && co0 + lc < d.Co) v = *reinterpret_cast<const float4 *>(dY + p * d.Co + co0 + lc);
-                As[lc + 0][pl] = f2bf(v.x);
-                As[lc + 1][pl] = f2bf(v.y);
-                As[lc + 2][pl] = f2bf(v.z);
-                As[lc + 3][pl] = f2bf(v.w);
-            }
-            {   // B: X(p, kq0+lc..+3) -> Bs[k][pix]
-                float4 v = {0.f, 0.f, 0.f, 0.f};
-                if (okp && kl < K) {
-                    const long long src = shifted_pixel(p, ltap, d.ks, d.H, d.W);
-                    v = *reinterpret_cast<const float4 *>(X + src * d.Ci + lci);
-                }
-                Bs[lc + 0][pl] = f2bf(v.x);
-                Bs[lc + 1][pl] = f2bf(v.y);
-                Bs[lc + 2][pl] = f2bf(v.z);
-                Bs[lc + 3][pl] = f2bf(v.w);
+            const int row = 4 * h + g;
+            const bf16x8 af = frag(&Ys[(row * CONV_P + l4) * WG_LD + (wave >> 1) * 16 + ch]);
+#pragma unroll
+            for (int k = 0; k < KS * KS; ++k) {
+                const bf16x8 bf = frag(&Xs[((row + k / KS) * R + l4 + k % KS) * WG_LD + (wave & 1) * 16 + ch]);
+                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bf, acc[k], 0, 0, 0);
             }
         }
-        __syncthreads();
-        bf16x8 af[2], bfm[2];
-        for (int a = 0; a < 2; ++a) {
-            const int row = wc + a * 16 + (lane & 15);
-            af[a] = *reinterpret_cast<const bf16x8 *>(&As[row][8 * (lane >> 4)]);
-        }
-        for (int b = 0; b < 2; ++b) {
-            const int col = wk + b * 16 + (lane & 15);
-            bfm[b] = *reinterpret_cast<const bf16x8 *>(&Bs[col][8 * (lane >> 4)]);
-        }
-        for (int a = 0; a < 2; ++a)
-            for (int b = 0; b < 2; ++b)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfm[b], acc[a][b], 0, 0, 0);
-        __syncthreads();
     }
-    float *pz = part + (long long)blockIdx.z * d.Co * K;
-    for (int a = 0; a < 2; ++a)
-        for (int b = 0; b < 2; ++b)
-            for (int i = 0; i < 4; ++i) {
-                const int co = co0 + wc + a * 16 + 4 * (lane >> 4) + i;
-                const int k = kq0 + wk + b * 16 + (lane & 15);
-                if (co < d.Co && k < K) pz[(long long)co * K + k] = acc[a][b][i];
-            }
+    const long long K = (long long)KS * KS * d.Ci;
+    float *pz = part + (long long)blockIdx.z * (d.Co * K + d.Co);
+    const int ci = ci0 + (wave & 1) * 16 + (lane & 15);
+    if (ci < d.Ci)
+#pragma unroll
+        for (int k = 0; k < KS * KS; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                pz[(co0 + (wave >> 1) * 16 + 4 * g + i) * K + k * d.Ci + ci] = acc[k][i];
+    if (blockIdx.x == 0) {
+        // a channel's 64 pixel sums in LDS, added in pixel order by one lane
+        __shared__ float bs[CONV_P * CONV_P][33];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) bs[t >> 2][8 * (t & 3) + c] = bsum[c];
+        __syncthreads();
+        if (t < 32) {
+            float s = 0.f;
+            for (int p = 0; p < CONV_P * CONV_P; ++p) s += bs[p][t];
+            pz[d.Co * K + co0 + t] = s;
+        }
+    }
 }
 
-__global__ void k_wgrad_reduce(const float *__restrict__ part, int nz, long long n, float *__restrict__ dW) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < nz; ++z) s += part[(long long)z * n + t];
-    dW[t] = s;
-}
-
-// bias gradient: db[co] = sum_p dY[p][co] (one block per channel, fixed order)
-__global__ __launch_bounds__(256) void k_bgrad(const float *__restrict__ dY, long long P, int Co,
-                                               float *__restrict__ db) {
-    __shared__ float red[256];
-    const int co = blockIdx.x;
-    float s = 0.f;
-    for (long long p = threadIdx.x; p < P; p += 256) s += dY[p * Co + co];
-    red[threadIdx.x] = s;
+// dW[e] = sum over the runs of part[run][e]: 64 entries a workgroup of NW waves, wave w on runs
+// 4 w .. 4 w + 3, then 4 NW further on (4 loads in flight a lane), the waves added in order.
+// 16 waves where there are many runs of a small layer (512 runs of 9,248 entries).
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_wgrad_reduce(const float *__restrict__ part, int runs, long long n,
+                                                          float *__restrict__ dW) {
+    __shared__ float red[NW][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long long e = (long long)blockIdx.x * 64 + lane;
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    if (e < n)
+        for (int z = 4 * w; z < runs; z += 4 * NW)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (z + u < runs) a[u] += part[(long long)(z + u) * n + e];
+    red[w][lane] = (a[0] + a[1]) + (a[2] + a[3]);
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    if (w == 0 && e < n) {
+        float s = red[0][lane];
+#pragma unroll
+        for (int v = 1; v < NW; ++v) s += red[v][lane];
+        dW[e] = s;
     }
-    if (threadIdx.x == 0) db[co] = red[0];
-}
-
-__global__ void k_relu_bwd(long long n, const float *__restrict__ y, float *__restrict__ dy) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n && !(y[t] > 0.f)) dy[t] = 0.f;
 }
 
 // 2x2 average pool and nearest 2x upsample, NHWC, with their adjoints
@@ -284,67 +358,56 @@ __global__ void k_pool(int B, int H, int W, int C, const float *__restrict__ in,
     out[t] = 0.25f * (at(2 * y, 2 * x) + at(2 * y, 2 * x + 1) + at(2 * y + 1, 2 * x) + at(2 * y + 1, 2 * x + 1));
 }
 
-__global__ void k_pool_bwd(int B, int H, int W, int C, const float *__restrict__ dout, float *__restrict__ din) {
-    const long long n = (long long)B * H * W * C;
+// gradient of an encoder output that feeds a 2x2 pool and, through the decoder's
+// concatenation, channels [Ca, Ca + C) of dcat: the sum of both, zero where the output y
+// (a ReLU's) is not positive
+__global__ void k_skip_bwd(int B, int H, int W, int C, int Ca, const float *__restrict__ dcat,
+                           const float *__restrict__ dpool, const float *__restrict__ y, float *__restrict__ dy) {
+    const long long n = (long long)B * H * W * (C / 4);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    const int c = (int)(t % C);
-    long long r = t / C;
-    const int x = (int)(r % W);
-    r /= W;
-    const int y = (int)(r % H);
+    const int c = (int)(t % (C / 4)) * 4;
+    const long long p = t / (C / 4);
+    const long long r = p / W;
+    const int x = (int)(p - r * W), yy = (int)(r % H);
     const long long b = r / H;
-    din[t] = 0.25f * dout[((b * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
+    const float4 a = *reinterpret_cast<const float4 *>(dcat + p * (Ca + C) + Ca + c);
+    const float4 q = *reinterpret_cast<const float4 *>(dpool + ((b * (H / 2) + yy / 2) * (W / 2) + x / 2) * C + c);
+    const float4 m = *reinterpret_cast<const float4 *>(y + p * C + c);
+    float4 o;
+    o.x = m.x > 0.f ? a.x + 0.25f * q.x : 0.f;
+    o.y = m.y > 0.f ? a.y + 0.25f * q.y : 0.f;
+    o.z = m.z > 0.f ? a.z + 0.25f * q.z : 0.f;
+    o.w = m.w > 0.f ? a.w + 0.25f * q.w : 0.f;
+    *reinterpret_cast<float4 *>(dy + p * C + c) = o;
 }
 
-// upsample a (H/2 x W/2, Ca) to H x W into channels [0, Ca) of out (Ctot) and copy
-// skip (H x W, Cs) into channels [Ca, Ca + Cs): the decoder's up + concat
-__global__ void k_up_cat(int B, int H, int W, int Ca, int Cs, const float *__restrict__ a,
-                         const float *__restrict__ skip, float *__restrict__ out) {
-    const int Ct = Ca + Cs;
-    const long long n = (long long)B * H * W * Ct;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int c = (int)(t % Ct);
-    const long long p = t / Ct;
-    if (c < Ca) {
-        const int x = (int)(p % W);
-        const long long r = p / W;
-        const int y = (int)(r % H);
-        const long long b = r / H;
-        out[t] = a[((b * (H / 2) + y / 2) * (W / 2) + x / 2) * Ca + c];
-    } else {
-        out[t] = skip[p * Cs + (c - Ca)];
-    }
-}
-
-// adjoint of k_up_cat: da (H/2 x W/2, Ca) = sum of the 4 children; dskip += tail
-__global__ void k_up_cat_bwd_a(int B, int H, int W, int Ca, int Cs, const float *__restrict__ dout,
-                               float *__restrict__ da) {
+// gradient of the low-resolution input of the decoder's up + concat: the sum over its 4
+// children of channels [0, Ca) of dcat, zero where the input y (a ReLU's) is not positive
+__global__ void k_up_cat_bwd(int B, int H, int W, int Ca, int Cs, const float *__restrict__ dcat,
+                             const float *__restrict__ y, float *__restrict__ da) {
     const int Ct = Ca + Cs, h = H / 2, w = W / 2;
-    const long long n = (long long)B * h * w * Ca;
+    const long long n = (long long)B * h * w * (Ca / 4);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    const int c = (int)(t % Ca);
-    long long r = t / Ca;
-    const int x = (int)(r % w);
-    r /= w;
-    const int y = (int)(r % h);
+    const int c = (int)(t % (Ca / 4)) * 4;
+    const long long p = t / (Ca / 4);
+    const long long r = p / w;
+    const int x = (int)(p - r * w), yy = (int)(r % h);
     const long long b = r / h;
-    float s = 0.f;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int dy = 0; dy < 2; ++dy)
-        for (int dx = 0; dx < 2; ++dx) s += dout[((b * H + 2 * y + dy) * W + 2 * x + dx) * Ct + c];
-    da[t] = s;
-}
-
-__global__ void k_up_cat_bwd_skip(long long P, int Ca, int Cs, const float *__restrict__ dout,
-                                  float *__restrict__ dskip) {
-    const long long n = P * Cs;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const long long p = t / Cs;
-    const int c = (int)(t % Cs);
-    dskip[t] += dout[p * (Ca + Cs) + Ca + c];
+        for (int dx = 0; dx < 2; ++dx) {
+            const float4 v = *reinterpret_cast<const float4 *>(
+                dcat + ((b * H + 2 * yy + dy) * W + 2 * x + dx) * Ct + c);
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
+    const float4 m = *reinterpret_cast<const float4 *>(y + p * Ca + c);
+    *reinterpret_cast<float4 *>(da + p * Ca + c) = make_float4(m.x > 0.f ? s.x : 0.f, m.y > 0.f ? s.y : 0.f,
+                                                               m.z > 0.f ? s.z : 0.f, m.w > 0.f ? s.w : 0.f);
 }
 
 // masked mean squared error over the SG_OUT used channels; out has SG_OUT_PAD channels
@@ -353,35 +416,38 @@ __global__ __launch_bounds__(256) void k_loss(long long P, int nch, const float 
                                               const float *__restrict__ mask,
                                               const float *__restrict__ chw,
                                               double *__restrict__ partials) {
-    __shared__ double red[256];
     double s = 0.0, m = 0.0;
-    for (long long p = (long long)blockIdx.x * 256 + threadIdx.x; p < P; p += (long long)gridDim.x * 256) {
+    // a lane per (pixel, channel) of the targets, so that a wave reads both images in runs
+    const long long n = P * SG_OUT, step = (long long)gridDim.x * 256;
+    for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < n; t += step) {
+        const long long p = t / SG_OUT;
+        const int c = (int)(t - p * SG_OUT);
         const float mk = mask[p];
         if (mk == 0.f) continue;
-        m += mk;
-        for (int c = 0; c < nch; ++c) {
-            const double e = (double)out[p * SG_OUT_PAD + c] - tgt[p * SG_OUT + c];
+        if (c == 0) m += mk;
+        if (c < nch) {
+            const double e = (double)out[p * SG_OUT_PAD + c] - tgt[t];
             s += mk * chw[c] * e * e;
         }
     }
-    for (int pass = 0; pass < 2; ++pass) {
-        red[threadIdx.x] = pass == 0 ? s : m;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) partials[2 * blockIdx.x + pass] = red[0];
-        __syncthreads();
-    }
+    double v[2] = {s, m};
+    block_reduce_store<2>(v, partials);
 }
 
-__global__ void k_loss_final(const double *__restrict__ partials, int nb, double *__restrict__ res) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0, m = 0.0;
-    for (int b = 0; b < nb; ++b) { s += partials[2 * b]; m += partials[2 * b + 1]; }
-    res[0] = m > 0 ? s / m : 0.0;
-    res[1] = m;
+__global__ __launch_bounds__(256) void k_loss_final(const double *__restrict__ partials, int nb,
+                                                    double *__restrict__ res) {
+    double v[2] = {0.0, 0.0};
+    for (int b = threadIdx.x; b < nb; b += 256) {
+        v[0] += partials[2 * b];
+        v[1] += partials[2 * b + 1];
+    }
+    __shared__ double tot[2];
+    block_reduce_store<2>(v, tot, 0);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        res[0] = tot[1] > 0 ? tot[0] / tot[1] : 0.0;
+        res[1] = tot[1];
+    }
 }
 
 __global__ void k_loss_grad(long long P, int nch, const float *__restrict__ out,
@@ -412,21 +478,34 @@ __global__ void k_adam(long long n, float *__restrict__ w, const float *__restri
     w[t] = w[t] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
 }
 
-// BF16 copy of the forward weights W[co][k] and of the data-gradient weights
-// W'[ci][k'] (k' = tap'*Co + co, tap' = 8 - tap): dX = conv(dY, W') with the
-// flipped kernel, periodic padding making it exact
+// BF16 copies of the weights in the order k_conv_patch reads them, [row / 16][k / 32][lane][8]
+// (lane l: row l & 15, k from 8 (l >> 4)), zeros past K: the forward weights W[co][k], and the
+// data gradient's W'[ci][k'] (k' = tap'*Co + co, tap' = 8 - tap): dX = conv(dY, W') with the
+// flipped kernel, periodic padding making it exact.  One lane per BF16 value of either copy.
+__host__ __device__ inline long long frag_size(int rows, int K) { return (long long)rows * ((K + 31) / 32 * 32); }
+
 __global__ void k_prep_weights(int Co, int Ci, int ks, const float *__restrict__ W,
-                               short *__restrict__ Wb, short *__restrict__ Wt) {
-    const int K = ks * ks * Ci;
-    const long long n = (long long)Co * K;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int co = (int)(t / K), k = (int)(t % K);
-    const int tap = k / Ci, ci = k % Ci;
-    const short b = f2bf(W[t]);
-    Wb[t] = b;
-    const int tapf = ks == 3 ? 8 - tap : 0;
-    Wt[(long long)ci * (ks * ks * Co) + (long long)tapf * Co + co] = b;
+                               short *__restrict__ Wf, short *__restrict__ Wt) {
+    const int kk = ks * ks;
+    const long long nf = frag_size(Co, kk * Ci), nt = frag_size(Ci, kk * Co);
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nf + nt) return;
+    const bool fwd = t < nf;
+    if (!fwd) t -= nf;
+    const int K = fwd ? kk * Ci : kk * Co, S = (K + 31) / 32;
+    const int j = (int)(t & 7), lane = (int)(t >> 3) & 63;
+    const long long f = t >> 9;
+    const int row = (int)(f / S) * 16 + (lane & 15), k = (int)(f % S) * 32 + 8 * (lane >> 4) + j;
+    short v = 0;
+    if (k < K) {
+        if (fwd) {
+            v = f2bf(W[(long long)row * K + k]);
+        } else {
+            const int tap = k / Co, co = k - tap * Co;
+            v = f2bf(W[((long long)co * kk + (ks == 3 ? 8 - tap : 0)) * Ci + row]);
+        }
+    }
+    (fwd ? Wf : Wt)[t] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -434,8 +513,9 @@ __global__ void k_prep_weights(int Co, int Ci, int ks, const float *__restrict__
 // ---------------------------------------------------------------------------
 struct ConvLayer {
     int ks, Ci, Co, relu;
-    long long woff, boff;   // offsets into the parameter vector
-    short *Wb, *Wt;         // BF16 forward / data-gradient weights
+    long long woff, boff;   // offsets into the parameter vector: the biases follow the weights
+    long long nparams() const { return (long long)Co * ks * ks * Ci + Co; }
+    short *Wf, *Wt;         // BF16 forward / data-gradient weights, as the MFMA reads them
 };
 
 struct Act {
@@ -458,7 +538,7 @@ struct cism_surrogate {
     hipStream_t stream;
     hipEvent_t ev0, ev1;
     float last_forward_ms;   // device time of the last forward pass (kernels only)
-    int wprep_ok;            // the BF16 copies Wb, Wt match w (cleared whenever w changes)
+    int wprep_ok;            // the BF16 copies Wf, Wt match w (cleared whenever w changes)
 };
 
 // activation indices
@@ -471,6 +551,18 @@ enum { L_E0a, L_E0b, L_E1a, L_E1b, L_E2a, L_E2b, L_M0, L_M1, L_D2, L_D1, L_D0, L
 
 static const int LAYER_IN[L_N] = {A_IN, A_E0a, A_P0, A_E1a, A_P1, A_E2a, A_P2, A_M0, A_C2, A_C1, A_C0, A_D0};
 static const int LAYER_OUT[L_N] = {A_E0a, A_E0b, A_E1a, A_E1b, A_E2a, A_E2b, A_M0, A_M1, A_D2, A_D1, A_D0, A_OUT};
+
+// the weight gradient's split of a layer's patches into runs of `per`: about 512 workgroups,
+// with at least 4 patches each so that the partials (Co * K floats a run) stay a small part
+// of the traffic
+static void wgrad_runs(const ConvLayer &c, int B, int H, int W, int &runs, int &per) {
+    const int np = B * ((H + CONV_P - 1) / CONV_P) * ((W + CONV_P - 1) / CONV_P);
+    const int tiles = ((c.Ci + 31) / 32) * (c.Co / 32);
+    int want = (512 + tiles - 1) / tiles;
+    if (want > (np + 3) / 4) want = (np + 3) / 4;
+    per = (np + want - 1) / want;
+    runs = (np + per - 1) / per;
+}
 
 static int sg_alloc(float **p, long long n) {
     hipError_t e = hipMalloc(p, sizeof(float) * (n > 0 ? n : 1));
@@ -505,7 +597,7 @@ extern "C" int cism_surrogate_create(int H, int W, int batch, int device, cism_s
         off += (long long)c.Co * c.ks * c.ks * c.Ci;
         c.boff = off;
         off += c.Co;
-        c.Wb = c.Wt = nullptr;
+        c.Wf = c.Wt = nullptr;
         s->L.push_back(c);
     }
     s->nparams = off;
@@ -523,13 +615,15 @@ extern "C" int cism_surrogate_create(int H, int W, int batch, int device, cism_s
         s->A.push_back(x);
     }
     for (int a = 0; a < A_N && !st; ++a) {
-        st = sg_alloc(&s->A[a].y, s->A[a].n(batch));
+        // the concatenations exist as gradients only: the convolutions read their parts
+        const bool cat = a == A_C0 || a == A_C1 || a == A_C2;
+        if (!cat) st = sg_alloc(&s->A[a].y, s->A[a].n(batch));
         if (!st) st = sg_alloc(&s->A[a].dy, s->A[a].n(batch));
     }
     for (int l = 0; l < L_N && !st; ++l) {
-        const long long nw = (long long)s->L[l].Co * s->L[l].ks * s->L[l].ks * s->L[l].Ci;
-        if (hipMalloc(&s->L[l].Wb, sizeof(short) * nw) != hipSuccess ||
-            hipMalloc(&s->L[l].Wt, sizeof(short) * nw) != hipSuccess)
+        const ConvLayer &c = s->L[l];
+        if (hipMalloc(&s->L[l].Wf, sizeof(short) * frag_size(c.Co, c.ks * c.ks * c.Ci)) != hipSuccess ||
+            hipMalloc(&s->L[l].Wt, sizeof(short) * frag_size(c.Ci, c.ks * c.ks * c.Co)) != hipSuccess)
             st = CISM_ERR_NOMEM;
     }
     if (!st) st = sg_alloc(&s->w, s->nparams);
@@ -541,10 +635,12 @@ extern "C" int cism_surrogate_create(int H, int W, int batch, int device, cism_s
     if (!st) st = sg_alloc(&s->tgt, P * SG_OUT);
     if (!st) st = sg_alloc(&s->mask, P);
     if (!st) st = sg_alloc(&s->chw, SG_OUT);
-    // weight-gradient partials: the largest Co*K times the pixel split
+    // weight-gradient partials: the largest layer's runs
     s->wpart_n = 0;
     for (int l = 0; l < L_N; ++l) {
-        const long long n = (long long)s->L[l].Co * s->L[l].ks * s->L[l].ks * s->L[l].Ci * 64;
+        int runs, per;
+        wgrad_runs(s->L[l], batch, s->A[LAYER_OUT[l]].H, s->A[LAYER_OUT[l]].W, runs, per);
+        const long long n = (long long)runs * s->L[l].nparams();
         if (n > s->wpart_n) s->wpart_n = n;
     }
     if (!st) st = sg_alloc(&s->wpart, s->wpart_n);
@@ -592,7 +688,7 @@ extern "C" int cism_surrogate_destroy(cism_surrogate *s) {
         if (a.dy) (void)hipFree(a.dy);
     }
     for (auto &l : s->L) {
-        if (l.Wb) (void)hipFree(l.Wb);
+        if (l.Wf) (void)hipFree(l.Wf);
         if (l.Wt) (void)hipFree(l.Wt);
     }
     void *ptrs[] = {s->w, s->g, s->m, s->v, s->raw, s->tgt, s->mask, s->chw, s->wpart, s->lpart, s->lres};
@@ -634,26 +730,46 @@ extern "C" int cism_surrogate_set_params(cism_surrogate *s, const float *host) {
 static int prep_weights(cism_surrogate *s) {
     if (s->wprep_ok) return CISM_OK;
     for (auto &c : s->L) {
-        const long long n = (long long)c.Co * c.ks * c.ks * c.Ci;
+        const long long n = frag_size(c.Co, c.ks * c.ks * c.Ci) + frag_size(c.Ci, c.ks * c.ks * c.Co);
         hipLaunchKernelGGL(k_prep_weights, dim3(nblocks_for(n)), dim3(256), 0, s->stream, c.Co, c.Ci, c.ks,
-                           s->w + c.woff, c.Wb, c.Wt);
+                           s->w + c.woff, c.Wf, c.Wt);
     }
     HIP_TRY(hipGetLastError());
     s->wprep_ok = 1;
     return CISM_OK;
 }
 
-static int conv_launch(cism_surrogate *s, const ConvDims &d, const float *in, const short *Wb,
-                       const float *bias, float *out) {
-    if (d.Ci % 16 != 0 || (d.ks != 1 && d.ks != 3)) {
-        cism_set_error("surrogate convolution: Ci %% 16 must be 0 and the kernel 1x1 or 3x3");
+static int conv_launch(cism_surrogate *s, const ConvDims &d, const ConvSrc &src, const short *Wf,
+                       const float *bias, const float *mask, float *out) {
+    if (d.Ci % 16 != 0 || d.Co % 32 != 0 || (d.ks != 1 && d.ks != 3)) {
+        cism_set_error("surrogate convolution: Ci %% 16 and Co %% 32 must be 0 and the kernel 1x1 or 3x3");
         return CISM_ERR_ARG;
     }
-    const long long P = (long long)d.B * d.H * d.W;
-    dim3 grid((unsigned)((P + 63) / 64), (unsigned)((d.Co + 63) / 64));
-    hipLaunchKernelGGL(k_conv_mfma, grid, dim3(256), 0, s->stream, d, in, Wb, bias, out);
+    const int R = CONV_P + (d.ks == 3 ? 2 : 0);
+    const size_t lds = sizeof(short) * R * R * (d.Ci + 8);   // at most 52.8 KB (256 channels)
+    const unsigned np = (unsigned)(d.B * ((d.H + CONV_P - 1) / CONV_P) * ((d.W + CONV_P - 1) / CONV_P));
+    // 64 output channels a workgroup read each staged patch half as often; 32 where that
+    // leaves fewer than two workgroups a CU
+    if (d.Co % 64 == 0 && np * (d.Co / 64) >= 512)
+        hipLaunchKernelGGL(k_conv_patch<2>, dim3(np, d.Co / 64), dim3(256), lds, s->stream, d, src, Wf, bias, mask,
+                           out);
+    else
+        hipLaunchKernelGGL(k_conv_patch<1>, dim3(np, d.Co / 32), dim3(256), lds, s->stream, d, src, Wf, bias, mask,
+                           out);
     HIP_TRY(hipGetLastError());
     return CISM_OK;
+}
+
+// what layer l reads
+static ConvSrc layer_src(const cism_surrogate *s, int l) {
+    auto cat = [&](int low, int skip) {
+        return ConvSrc{s->A[low].y, s->A[skip].y, s->A[low].C, s->A[skip].C};
+    };
+    if (l == L_D2) return cat(A_M1, A_E2b);
+    if (l == L_D1) return cat(A_D2, A_E1b);
+    if (l == L_D0) return cat(A_D1, A_E0b);
+    const Act &in = s->A[LAYER_IN[l]];
+    return ConvSrc{in.y, nullptr, in.C, 0};
 }
 
 static int forward(cism_surrogate *s) {
@@ -661,125 +777,87 @@ static int forward(cism_surrogate *s) {
     CISM_TRY(prep_weights(s));
     auto conv = [&](int l) -> int {
         const ConvLayer &c = s->L[l];
-        const Act &in = s->A[LAYER_IN[l]], &out = s->A[LAYER_OUT[l]];
-        ConvDims d = {B, in.H, in.W, c.Ci, c.Co, c.ks, c.relu};
-        return conv_launch(s, d, in.y, c.Wb, s->w + c.boff, out.y);
+        const Act &out = s->A[LAYER_OUT[l]];
+        ConvDims d = {B, out.H, out.W, c.Ci, c.Co, c.ks, c.relu};
+        return conv_launch(s, d, layer_src(s, l), c.Wf, s->w + c.boff, nullptr, out.y);
     };
     auto pool = [&](int a_in, int a_out) {
         const Act &x = s->A[a_in];
         hipLaunchKernelGGL(k_pool, dim3(nblocks_for(s->A[a_out].n(B))), dim3(256), 0, s->stream, B, x.H, x.W,
                            x.C, x.y, s->A[a_out].y);
     };
-    auto upcat = [&](int a_low, int a_skip, int a_out) {
-        const Act &o = s->A[a_out];
-        hipLaunchKernelGGL(k_up_cat, dim3(nblocks_for(o.n(B))), dim3(256), 0, s->stream, B, o.H, o.W,
-                           s->A[a_low].C, s->A[a_skip].C, s->A[a_low].y, s->A[a_skip].y, o.y);
-    };
     CISM_TRY(conv(L_E0a)); CISM_TRY(conv(L_E0b)); pool(A_E0b, A_P0);
     CISM_TRY(conv(L_E1a)); CISM_TRY(conv(L_E1b)); pool(A_E1b, A_P1);
     CISM_TRY(conv(L_E2a)); CISM_TRY(conv(L_E2b)); pool(A_E2b, A_P2);
     CISM_TRY(conv(L_M0)); CISM_TRY(conv(L_M1));
-    upcat(A_M1, A_E2b, A_C2); CISM_TRY(conv(L_D2));
-    upcat(A_D2, A_E1b, A_C1); CISM_TRY(conv(L_D1));
-    upcat(A_D1, A_E0b, A_C0); CISM_TRY(conv(L_D0));
+    CISM_TRY(conv(L_D2)); CISM_TRY(conv(L_D1)); CISM_TRY(conv(L_D0));
     CISM_TRY(conv(L_HEAD));
     HIP_TRY(hipGetLastError());
     return CISM_OK;
 }
 
-// backward of layer l given dY of its output (already ReLU-masked); adds dX into the
-// input activation's gradient when want_dx
-static int conv_backward(cism_surrogate *s, int l, bool want_dx) {
+// backward of layer l given dY of its output (already ReLU-masked): its parameter gradients
+// and, when want_dx, the gradient of its input, zeroed where mask (the input itself, when
+// it is a ReLU's output used by this layer alone) is not positive
+static int conv_backward(cism_surrogate *s, int l, bool want_dx, bool mask) {
     const int B = s->B;
     const ConvLayer &c = s->L[l];
     const Act &in = s->A[LAYER_IN[l]], &out = s->A[LAYER_OUT[l]];
-    const long long P = (long long)B * in.H * in.W;
-    const int K = c.ks * c.ks * c.Ci;
-    // weight gradient
-    int nzs = (int)((P + 4095) / 4096);
-    if (nzs > 64) nzs = 64;
-    const long long pchunk = ((P + nzs - 1) / nzs + 15) / 16 * 16;
-    ConvDims d = {B, in.H, in.W, c.Ci, c.Co, c.ks, 0};
-    dim3 grid((unsigned)((K + 63) / 64), (unsigned)((c.Co + 63) / 64), (unsigned)nzs);
-    hipLaunchKernelGGL(k_wgrad_mfma, grid, dim3(256), 0, s->stream, d, out.dy, in.y, s->wpart, pchunk);
-    const long long nw = (long long)c.Co * K;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(nblocks_for(nw)), dim3(256), 0, s->stream, s->wpart, nzs, nw,
-                       s->g + c.woff);
-    hipLaunchKernelGGL(k_bgrad, dim3(c.Co), dim3(256), 0, s->stream, out.dy, P, c.Co, s->g + c.boff);
+    int runs, per;
+    wgrad_runs(c, B, out.H, out.W, runs, per);
+    ConvDims d = {B, out.H, out.W, c.Ci, c.Co, c.ks, 0};
+    const dim3 grid((unsigned)((c.Ci + 31) / 32), (unsigned)(c.Co / 32), (unsigned)runs);
+    hipLaunchKernelGGL(c.ks == 3 ? k_wgrad_patch<3> : k_wgrad_patch<1>, grid, dim3(256), 0, s->stream, d,
+                       layer_src(s, l), out.dy, s->wpart, per);
+    const dim3 gred((unsigned)((c.nparams() + 63) / 64));
+    if (runs > 64)
+        hipLaunchKernelGGL(k_wgrad_reduce<16>, gred, dim3(1024), 0, s->stream, s->wpart, runs, c.nparams(),
+                           s->g + c.woff);
+    else
+        hipLaunchKernelGGL(k_wgrad_reduce<4>, gred, dim3(256), 0, s->stream, s->wpart, runs, c.nparams(),
+                           s->g + c.woff);
     HIP_TRY(hipGetLastError());
     if (want_dx) {
         // dX = conv(dY, W') : channels Co -> Ci
-        ConvDims dd = {B, in.H, in.W, c.Co, c.Ci, c.ks, 0};
-        CISM_TRY(conv_launch(s, dd, out.dy, c.Wt, nullptr, in.dy));
+        ConvDims dd = {B, out.H, out.W, c.Co, c.Ci, c.ks, 0};
+        CISM_TRY(conv_launch(s, dd, ConvSrc{out.dy, nullptr, c.Co, 0}, c.Wt, nullptr, mask ? in.y : nullptr, in.dy));
     }
     return CISM_OK;
 }
 
 static int backward(cism_surrogate *s) {
     const int B = s->B;
-    auto relu_bwd = [&](int a) {
-        const Act &x = s->A[a];
-        hipLaunchKernelGGL(k_relu_bwd, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream, x.n(B), x.y, x.dy);
-    };
+    // the low-resolution input of a concatenation
     auto upcat_bwd = [&](int a_low, int a_skip, int a_cat) {
-        // d(low) = sum of children of the first channels; d(skip) += tail channels
-        const Act &o = s->A[a_cat];
-        hipLaunchKernelGGL(k_up_cat_bwd_a, dim3(nblocks_for(s->A[a_low].n(B))), dim3(256), 0, s->stream, B,
-                           o.H, o.W, s->A[a_low].C, s->A[a_skip].C, o.dy, s->A[a_low].dy);
-        hipLaunchKernelGGL(k_up_cat_bwd_skip, dim3(nblocks_for(s->A[a_skip].n(B))), dim3(256), 0, s->stream,
-                           (long long)B * o.H * o.W, s->A[a_low].C, s->A[a_skip].C, o.dy, s->A[a_skip].dy);
+        const Act &o = s->A[a_cat], &low = s->A[a_low];
+        hipLaunchKernelGGL(k_up_cat_bwd, dim3(nblocks_for(low.n(B) / 4)), dim3(256), 0, s->stream, B, o.H, o.W, low.C,
+                           s->A[a_skip].C, o.dy, low.y, low.dy);
     };
-    // head: dOUT set by the loss
-    CISM_TRY(conv_backward(s, L_HEAD, true));          // -> dD0
-    relu_bwd(A_D0); CISM_TRY(conv_backward(s, L_D0, true));   // -> dC0
-    upcat_bwd(A_D1, A_E0b, A_C0);                       // dD1 = up^T, dE0b (skip) = tail (added below)
-    relu_bwd(A_D1); CISM_TRY(conv_backward(s, L_D1, true));   // -> dC1
+    // an encoder output, from the concatenation and from the pool after it
+    auto skip_bwd = [&](int a_low, int a, int a_cat, int a_pool) {
+        const Act &x = s->A[a];
+        hipLaunchKernelGGL(k_skip_bwd, dim3(nblocks_for(x.n(B) / 4)), dim3(256), 0, s->stream, B, x.H, x.W, x.C,
+                           s->A[a_low].C, s->A[a_cat].dy, s->A[a_pool].dy, x.y, x.dy);
+    };
+    CISM_TRY(conv_backward(s, L_HEAD, true, true));     // dOUT set by the loss -> dD0
+    CISM_TRY(conv_backward(s, L_D0, true, false));      // -> dC0
+    upcat_bwd(A_D1, A_E0b, A_C0);
+    CISM_TRY(conv_backward(s, L_D1, true, false));      // -> dC1
     upcat_bwd(A_D2, A_E1b, A_C1);
-    relu_bwd(A_D2); CISM_TRY(conv_backward(s, L_D2, true));   // -> dC2
+    CISM_TRY(conv_backward(s, L_D2, true, false));      // -> dC2
     upcat_bwd(A_M1, A_E2b, A_C2);
-    relu_bwd(A_M1); CISM_TRY(conv_backward(s, L_M1, true));   // -> dM0
-    relu_bwd(A_M0); CISM_TRY(conv_backward(s, L_M0, true));   // -> dP2
-    // dE2b = pool^T dP2 + skip part; the skip part was added by upcat_bwd into dE2b
-    // before pool_bwd would overwrite it, so accumulate via a temporary: pool_bwd
-    // writes into dE2a's buffer first (free at this point), then add
-    {
-        const Act &x = s->A[A_E2b];
-        float *tmp = s->A[A_E2a].dy;
-        hipLaunchKernelGGL(k_pool_bwd, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream, B, x.H, x.W, x.C,
-                           s->A[A_P2].dy, tmp);
-        hipLaunchKernelGGL(k_up_cat_bwd_skip, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream,
-                           (long long)B * x.H * x.W, 0, x.C, tmp, x.dy);
-    }
-    relu_bwd(A_E2b); CISM_TRY(conv_backward(s, L_E2b, true));   // -> dE2a
-    relu_bwd(A_E2a); CISM_TRY(conv_backward(s, L_E2a, true));   // -> dP1
-    {
-        const Act &x = s->A[A_E1b];
-        float *tmp = s->A[A_E1a].dy;
-        hipLaunchKernelGGL(k_pool_bwd, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream, B, x.H, x.W, x.C,
-                           s->A[A_P1].dy, tmp);
-        hipLaunchKernelGGL(k_up_cat_bwd_skip, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream,
-                           (long long)B * x.H * x.W, 0, x.C, tmp, x.dy);
-    }
-    relu_bwd(A_E1b); CISM_TRY(conv_backward(s, L_E1b, true));
-    relu_bwd(A_E1a); CISM_TRY(conv_backward(s, L_E1a, true));   // -> dP0
-    {
-        const Act &x = s->A[A_E0b];
-        float *tmp = s->A[A_E0a].dy;
-        hipLaunchKernelGGL(k_pool_bwd, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream, B, x.H, x.W, x.C,
-                           s->A[A_P0].dy, tmp);
-        hipLaunchKernelGGL(k_up_cat_bwd_skip, dim3(nblocks_for(x.n(B))), dim3(256), 0, s->stream,
-                           (long long)B * x.H * x.W, 0, x.C, tmp, x.dy);
-    }
-    relu_bwd(A_E0b); CISM_TRY(conv_backward(s, L_E0b, true));
-    relu_bwd(A_E0a); CISM_TRY(conv_backward(s, L_E0a, false));
+    CISM_TRY(conv_backward(s, L_M1, true, true));       // -> dM0
+    CISM_TRY(conv_backward(s, L_M0, true, false));      // -> dP2
+    skip_bwd(A_M1, A_E2b, A_C2, A_P2);
+    CISM_TRY(conv_backward(s, L_E2b, true, true));      // -> dE2a
+    CISM_TRY(conv_backward(s, L_E2a, true, false));     // -> dP1
+    skip_bwd(A_D2, A_E1b, A_C1, A_P1);
+    CISM_TRY(conv_backward(s, L_E1b, true, true));
+    CISM_TRY(conv_backward(s, L_E1a, true, false));     // -> dP0
+    skip_bwd(A_D1, A_E0b, A_C0, A_P0);
+    CISM_TRY(conv_backward(s, L_E0b, true, true));
+    CISM_TRY(conv_backward(s, L_E0a, false, false));
     HIP_TRY(hipGetLastError());
-    return CISM_OK;
-}
-
-static int zero_skip_grads(cism_surrogate *s) {
-    // the skip activations accumulate gradient from two paths
-    const int sk[3] = {A_E0b, A_E1b, A_E2b};
-    for (int a : sk) HIP_TRY(hipMemsetAsync(s->A[a].dy, 0, sizeof(float) * s->A[a].n(s->B), s->stream));
     return CISM_OK;
 }
 
@@ -805,11 +883,10 @@ static int upload_batch(cism_surrogate *s, const float *in, const float *tgt, co
 
 static int loss_and_grad(cism_surrogate *s, int nch, double *loss) {
     const long long P = (long long)s->B * s->H * s->W;
-    int nb = (int)((P + 255) / 256);
-    if (nb > 1024) nb = 1024;
+    const int nb = (int)(P * SG_OUT < 1024 * 256 ? (P * SG_OUT + 255) / 256 : 1024);
     hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, s->stream, P, nch, s->A[A_OUT].y, s->tgt, s->mask,
                        s->chw, s->lpart);
-    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(1), 0, s->stream, s->lpart, nb, s->lres);
+    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(256), 0, s->stream, s->lpart, nb, s->lres);
     hipLaunchKernelGGL(k_loss_grad, dim3(nblocks_for(P * SG_OUT_PAD)), dim3(256), 0, s->stream, P, nch,
                        s->A[A_OUT].y, s->tgt, s->mask, s->chw, s->lres, s->A[A_OUT].dy);
     HIP_TRY(hipGetLastError());
@@ -851,7 +928,6 @@ extern "C" int cism_surrogate_loss_grad(cism_surrogate *s, const float *in, cons
     CISM_TRY(upload_batch(s, in, tgt, mask));
     CISM_TRY(forward(s));
     CISM_TRY(loss_and_grad(s, nch, loss));
-    CISM_TRY(zero_skip_grads(s));
     CISM_TRY(backward(s));
     if (grad) {
         HIP_TRY(hipMemcpyAsync(grad, s->g, sizeof(float) * s->nparams, hipMemcpyDeviceToHost, s->stream));
