@@ -308,6 +308,25 @@ struct DepthDev {
     double *efvs3, *eqp, *omk, *om;
 };
 
+// value of lane P of the quad
+template <int P>
+__device__ __forceinline__ double quad_lane(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), P * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), P * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// the sum over the quad's points in their order
+__device__ __forceinline__ double quad_sum(double v) {
+    return quad_lane<0>(v) + quad_lane<1>(v) + quad_lane<2>(v) + quad_lane<3>(v);
+}
+
+// Four lanes a cell, lane p at quadrature point p: the point's layers and element terms are one
+// lane's work, the sums over the points are quad sums in point order (the values of one lane
+// that runs the points in turn), and the layer fields leave through LDS in contiguous runs.
+// Bound: the FP64 powers and divisions, 40 of each a cell and 10 layers.  A lane per cell left
+// one wave a SIMD and each layer field in steps of 80 to 320 bytes: DIVA, 516 x 516 cells, 10
+// layers 546 us, 199 here.
+#define DEPTH_CELLS 64   // cells a workgroup
 template <int APPROX>
 __global__ __launch_bounds__(256) void k_element_depth(GridDev g, DepthDev d, const int32_t *__restrict__ ac,
                                                        const double *__restrict__ xV,
@@ -316,50 +335,48 @@ __global__ __launch_bounds__(256) void k_element_depth(GridDev g, DepthDev d, co
                                                        const double *__restrict__ sthck, int whichefvs,
                                                        double efvs_constant, double *__restrict__ Ke,
                                                        DevScal *__restrict__ sc) {
-    const long long cell = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= (long long)g.nx * g.ny) return;
+    extern __shared__ double lay[];   // [cell][nz3]: first efvs of the layers, then omega_k
+    const long long ncell = (long long)g.nx * g.ny, cell0 = (long long)blockIdx.x * DEPTH_CELLS;
+    const int lc = threadIdx.x >> 2, p = threadIdx.x & 3;
+    const long long cell = cell0 + lc;
+    const int cells = (int)(ncell - cell0 < DEPTH_CELLS ? ncell - cell0 : DEPTH_CELLS);
     const int i = (int)(cell % g.nx) + 1, j = (int)(cell / g.nx) + 1;   // 1-based
-    const int L = d.nz3 - 1;
+    const int nz3 = d.nz3, L = nz3 - 1;
     const long long ncol = (long long)g.sx * g.sy;
-    double *ef = d.efvs3 + (long long)L * cell;
-    const bool ok = i >= CISM_NHALO + 1 && i <= g.nx - CISM_NHALO + 1 && j >= CISM_NHALO + 1 &&
+    const bool ok = lc < cells && i >= CISM_NHALO + 1 && i <= g.nx - CISM_NHALO + 1 && j >= CISM_NHALO + 1 &&
                     j <= g.ny - CISM_NHALO + 1 && ac[cell] != 0;
+    double *ml = lay + lc * nz3;
+    double *eq = d.eqp + (long long)L * (4 * cell + p);
+    // run [0, n) of the cells' layer rows to out (rows of w values)
+    auto flush = [&](double *__restrict__ out, int w) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < cells * w; t += 256) out[w * cell0 + t] = lay[t / w * nz3 + t % w];
+        __syncthreads();
+    };
     if (!ok) {
-        for (int k = 0; k < L; ++k) ef[k] = 0.0;
-        if (APPROX == 4) {
-            for (int k = 0; k <= L; ++k) d.omk[k + (long long)d.nz3 * cell] = 0.0;
-            d.om[cell] = 0.0;
+        if (lc < cells)
+            for (int k = p; k < nz3; k += 4) ml[k] = 0.0;
+    } else {
+        double x[4], y[4], u[4], v[4], hn[4], sx[4], sy[4], bx[4], by[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const long long vtx = (i - 1 + c_di2[n]) + (long long)g.sx * (j - 1 + c_dj2[n]);
+            x[n] = xV[vtx];
+            y[n] = yV[vtx];
+            u[n] = vel[2 * vtx];
+            v[n] = vel[2 * vtx + 1];
+            hn[n] = sthck[vtx];
+            if (APPROX == 3) {
+                sx[n] = d.dsdx[vtx];
+                sy[n] = d.dsdy[vtx];
+            } else {
+                bx[n] = d.btr[vtx];
+                by[n] = d.btr[ncol + vtx];
+            }
         }
-        return;
-    }
-    double x[4], y[4], u[4], v[4], hn[4], sx[4], sy[4], bx[4], by[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-        const long long vtx = (i - 1 + c_di2[n]) + (long long)g.sx * (j - 1 + c_dj2[n]);
-        x[n] = xV[vtx];
-        y[n] = yV[vtx];
-        u[n] = vel[2 * vtx];
-        v[n] = vel[2 * vtx + 1];
-        hn[n] = sthck[vtx];
-        if (APPROX == 3) {
-            sx[n] = d.dsdx[vtx];
-            sy[n] = d.dsdy[vtx];
-        } else {
-            bx[n] = d.btr[vtx];
-            by[n] = d.btr[ncol + vtx];
-        }
-    }
-    const double *fl = d.flwa + (long long)L * cell, *ff = d.ff3 + (long long)L * cell;
-    double *eq = d.eqp + (long long)L * 4 * cell;
-    for (int k = 0; k < L; ++k) ef[k] = 0.0;
-    double Kuu[10], Kvv[10], Kuv[16];
-#pragma unroll
-    for (int e = 0; e < 10; ++e) Kuu[e] = Kvv[e] = 0.0;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) Kuv[e] = 0.0;
-    const double r = 1.0 / sqrt(3.0);
-    const double p_eff = (1.0 - 3.0) / 3.0, p2 = p_eff / 2, emin = 1.0e-8;
-    for (int p = 0; p < 4; ++p) {
+        const double *fl = d.flwa + (long long)L * cell, *ff = d.ff3 + (long long)L * cell;
+        const double r = 1.0 / sqrt(3.0);
+        const double p_eff = (1.0 - 3.0) / 3.0, p2 = p_eff / 2, emin = 1.0e-8;
         const double xq = (p == 0 || p == 3) ? -r : r, yq = p < 2 ? -r : r;
         double dxr[4], dyr[4], phi[4];
         dxr[0] = -(1.0 - yq) / 4.0; dxr[1] = (1.0 - yq) / 4.0;
@@ -433,62 +450,64 @@ __global__ __launch_bounds__(256) void k_element_depth(GridDev g, DepthDev d, co
                 e = 1.0 / (2.0 * fl[k] * (tp * tp + tau_perp * tau_perp));
             } else {
                 // compute_effective_viscosity_diva (no cubic): vertical shear from the old efvs
-                double eo = eq[k + (long long)L * p];
+                double eo = eq[k];
                 if (eo == 0.0) eo = ff[k] * pow(emin, p_eff);
                 const double ss = (d.sigma[k] + d.sigma[k + 1]) / 2.0;
                 const double uz = tx * ss / eo, vz = ty * ss / eo;
                 const double sq = hsq + 0.25 * (uz * uz + vz * vz);
                 e = ff[k] * pow(sq, p2);
             }
-            if (APPROX == 4) eq[k + (long long)L * p] = e;
-            ef[k] = ef[k] + e;
+            if (APPROX == 4) eq[k] = e;
+            const double es = quad_sum(e) / 4;
+            if ((k & 3) == p) ml[k] = es;
             avg = avg + e * (d.sigma[k + 1] - d.sigma[k]);
         }
         double hq = 0.0;
 #pragma unroll
         for (int n = 0; n < 4; ++n) hq = hq + phi[n] * hn[n];
         const double f = hq * avg * 1.0 * det / CISM_VOL0;
+        // the quad's sums, entry by entry; lane p stores every fourth
+        auto entry = [&](int ent, double term) {
+            const double sum = quad_sum(term);
+            if ((ent & 3) == p) Ke[ke2idx(ent, cell)] = sum;
+        };
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
             for (int b = a; b < 4; ++b) {
-                Kuu[tri4(a, b)] = Kuu[tri4(a, b)] + f * (4.0 * dx[a] * dx[b] + dy[a] * dy[b] + 0.0 * 0.0);
-                Kvv[tri4(a, b)] = Kvv[tri4(a, b)] + f * (4.0 * dy[a] * dy[b] + dx[a] * dx[b] + 0.0 * 0.0);
+                entry(tri4(a, b), f * (4.0 * dx[a] * dx[b] + dy[a] * dy[b] + 0.0 * 0.0));
+                entry(10 + tri4(a, b), f * (4.0 * dy[a] * dy[b] + dx[a] * dx[b] + 0.0 * 0.0));
             }
 #pragma unroll
         for (int nc = 0; nc < 4; ++nc)
 #pragma unroll
             for (int nr = 0; nr < 4; ++nr)
-                Kuv[nr + 4 * nc] = Kuv[nr + 4 * nc] + f * (2.0 * dx[nr] * dy[nc] + dy[nr] * dx[nc]);
+                entry(20 + nr + 4 * nc, f * (2.0 * dx[nr] * dy[nc] + dy[nr] * dx[nc]));
     }
-    for (int k = 0; k < L; ++k) ef[k] = ef[k] / 4;
+    flush(d.efvs3, L);
     if (APPROX == 4) {
         // compute_integrals_diva: omega_k from the surface down, per quadrature point, then
         // their mean; omega the trapezoid integral of omega_k
-        double o0 = 0.0, o1 = 0.0, o2 = 0.0, o3 = 0.0;
-        double *ok = d.omk + (long long)d.nz3 * cell;
-        ok[L] = (o0 + o1 + o2 + o3) / 4;
-        const double H = d.thck[cell];
-        for (int k = L - 1; k >= 0; --k) {
-            const double depth = 0.5 * (d.sigma[k] + d.sigma[k + 1]);
-            const double dz = (d.sigma[k + 1] - d.sigma[k]) * H;
-            o0 = o0 + depth / eq[k] * dz;
-            o1 = o1 + depth / eq[k + L] * dz;
-            o2 = o2 + depth / eq[k + 2LL * L] * dz;
-            o3 = o3 + depth / eq[k + 3LL * L] * dz;
-            ok[k] = (o0 + o1 + o2 + o3) / 4;
+        if (ok) {
+            const double H = d.thck[cell];
+            double o = 0.0;
+            if (p == 0) ml[L] = 0.0;
+            for (int k = L - 1; k >= 0; --k) {
+                const double depth = 0.5 * (d.sigma[k] + d.sigma[k + 1]);
+                const double dz = (d.sigma[k + 1] - d.sigma[k]) * H;
+                o = o + depth / eq[k] * dz;
+                const double om = quad_sum(o) / 4;
+                if ((k & 3) == p) ml[k] = om;
+            }
         }
-        double om = 0.0;
-        for (int k = 0; k < L; ++k) om = om + 0.5 * (ok[k] + ok[k + 1]) * (d.sigma[k + 1] - d.sigma[k]);
-        d.om[cell] = om;
+        flush(d.omk, nz3);
+        if (p == 0 && lc < cells) {
+            double om = 0.0;
+            if (ok)
+                for (int k = 0; k < L; ++k) om = om + 0.5 * (ml[k] + ml[k + 1]) * (d.sigma[k + 1] - d.sigma[k]);
+            d.om[cell] = om;
+        }
     }
-#pragma unroll
-    for (int e = 0; e < 10; ++e) {
-        Ke[ke2idx(e, cell)] = Kuu[e];
-        Ke[ke2idx(10 + e, cell)] = Kvv[e];
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) Ke[ke2idx(20 + e, cell)] = Kuv[e];
 }
 
 // parallel_halo of a cell field (parallel_slap.F90:1794-1860), nhalo = 2: periodic
@@ -536,7 +555,9 @@ __global__ __launch_bounds__(256) void k_beta_eff(GridDev g, const double *__res
 
 // DIVA after each solve (velo_higher:3661-3700): basal traction beta_eff u on every
 // vertex; on active vertices the bed velocity u - tau_b stag_omega and the levels above
-// u_b + tau_b stag_omega_k(k) (compute_3d_velocity_diva, diva_level_index = 0)
+// u_b + tau_b stag_omega_k(k) (compute_3d_velocity_diva, diva_level_index = 0).  One lane per
+// level of a vertex, so that omega_k and the velocity move in runs (515 x 515 x 11: 31 us, 119 with
+// a lane per vertex).
 __global__ __launch_bounds__(256) void k_diva_velocity(GridDev g, int nz3, const double *__restrict__ omk,
                                                        const int32_t *__restrict__ ipl,
                                                        const int32_t *__restrict__ av,
@@ -544,23 +565,27 @@ __global__ __launch_bounds__(256) void k_diva_velocity(GridDev g, int nz3, const
                                                        const double *__restrict__ som,
                                                        const double *__restrict__ vel, double *__restrict__ btr,
                                                        double *__restrict__ u3, double *__restrict__ v3) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long ncol = (long long)g.sx * g.sy;
-    if (q >= ncol) return;
+    if (t >= ncol * nz3) return;
+    const long long q = t / nz3;
+    const int k = (int)(t - q * nz3);
     const int i = (int)(q % g.sx), j = (int)(q / g.sx);
     const double u2 = vel[2 * q], v2 = vel[2 * q + 1];
     const double tx = beff[q] * u2, ty = beff[q] * v2;
-    btr[q] = tx;
-    btr[ncol + q] = ty;
+    if (k == nz3 - 1) {
+        btr[q] = tx;
+        btr[ncol + q] = ty;
+    }
     if (!av[q]) return;
     const double ub = u2 - tx * som[q], vb = v2 - ty * som[q];
-    double *uc = u3 + (long long)nz3 * q, *vc = v3 + (long long)nz3 * q;
-    uc[nz3 - 1] = ub;
-    vc[nz3 - 1] = vb;
-    for (int k = 0; k < nz3 - 1; ++k) {
+    if (k == nz3 - 1) {
+        u3[t] = ub;
+        v3[t] = vb;
+    } else {
         const double sk = stagger_m1(g.nx, omk, ipl, i, j, nz3, k);
-        uc[k] = ub + tx * sk;
-        vc[k] = vb + ty * sk;
+        u3[t] = ub + tx * sk;
+        v3[t] = vb + ty * sk;
     }
 }
 
@@ -821,11 +846,12 @@ int assemble_depth_device(cism_ctx *c, int approx, int whichefvs, double efvs_co
     const GridDev &g = c->g;
     const long long ncell = (long long)g.nx * g.ny, ncol = (long long)g.sx * g.sy;
     const DepthDev d = depth_dev(c);
+    const size_t lds = sizeof(double) * DEPTH_CELLS * d.nz3;   // nz3 <= 64 (the entry point): 32 KB
     if (approx == 3)
-        hipLaunchKernelGGL(k_element_depth<3>, dim3(nblocks_for(ncell)), dim3(256), 0, c->stream, g, d, c->ac,
+        hipLaunchKernelGGL(k_element_depth<3>, dim3(nblocks_for(ncell, DEPTH_CELLS)), dim3(256), lds, c->stream, g, d, c->ac,
                            c->xV, c->yV, c->x, c->sthck, whichefvs, efvs_constant, c->ssa_Ke, c->sc);
     else
-        hipLaunchKernelGGL(k_element_depth<4>, dim3(nblocks_for(ncell)), dim3(256), 0, c->stream, g, d, c->ac,
+        hipLaunchKernelGGL(k_element_depth<4>, dim3(nblocks_for(ncell, DEPTH_CELLS)), dim3(256), lds, c->stream, g, d, c->ac,
                            c->xV, c->yV, c->x, c->sthck, whichefvs, efvs_constant, c->ssa_Ke, c->sc);
     HIP_TRY(hipGetLastError());
     if (approx == 4) {
@@ -852,7 +878,7 @@ int diva_post_solve_device(cism_ctx *c) {
     const GridDev &g = c->g;
     const long long ncol = (long long)g.sx * g.sy;
     const int nz3 = c->dep_nz3;
-    hipLaunchKernelGGL(k_diva_velocity, dim3(nblocks_for(ncol)), dim3(256), 0, c->stream, g, nz3, c->dep_omk,
+    hipLaunchKernelGGL(k_diva_velocity, dim3(nblocks_for(ncol * nz3)), dim3(256), 0, c->stream, g, nz3, c->dep_omk,
                        c->dep_ipl, c->av, c->dep_beff, c->dep_som, c->x, c->dep_btr, c->dep_u3, c->dep_v3);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(k_halo_lead, dim3(nblocks_for(ncol * nz3)), dim3(256), 0, c->stream, g, nz3, c->dep_u3);
