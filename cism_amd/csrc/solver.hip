@@ -1206,6 +1206,35 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
     if (want_rr) block_reduce_store<1>(acc, partials);
 }
 
+// The same on a one-level grid (the depth-integrated solvers), where the column solve is one
+// division: a lane per node and no LDS.  k_cg_update_sia has 64 nodes for its 256 lanes there
+// (515 x 515 columns: 17.7 us, 10.1 here).
+template <typename T>
+__global__ __launch_bounds__(CISM_BLOCK) void k_cg_update_level(GridDev g, T *z, const T *__restrict__ Az,
+                                                                T *__restrict__ d, T *__restrict__ qv,
+                                                                T *__restrict__ x, T *__restrict__ r, RedSrc src,
+                                                                DevScal *__restrict__ sc, int cur, int first,
+                                                                int zero_stop, const int32_t *__restrict__ av,
+                                                                const T *__restrict__ F) {
+    using V2 = typename Vec2<T>::t;
+    const long long ncol = (long long)g.sx * g.sy;
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool solve = q < ncol && av[q];
+    // the column factors sb(0) = 0 and gamma(0) = 0; beta(0) of u and v (k_sia_setup)
+    T bu = (T)1, bv = (T)1;
+    if (solve) {
+        bu = F[2 * ncol + q];
+        bv = F[3 * ncol + q];
+    }
+    double alpha, beta;
+    cg_scalars(src, sc, cur, first, zero_stop, alpha, beta);
+    if (q >= ncol) return;
+    const int j = (int)(q / g.sx), i = (int)(q - (long long)j * g.sx);
+    V2 rr;
+    const int st = cg_update_node<T>(g, q, 0, q, i, j, z, Az, d, qv, x, r, (T)alpha, (T)beta, first, av, rr);
+    if (st && solve) store2<T>(z, q, rr.x / bu, rr.y / bv);
+}
+
 // ---------------------------------------------------------------------------
 // PCG drivers
 // ---------------------------------------------------------------------------
@@ -1241,10 +1270,17 @@ struct CGVecs {
 // blocks of the fused update (one per 64 columns)
 static inline int sia_blocks(const GridDev &g) { return (int)(((long long)g.sx * g.sy + 63) / 64); }
 
+// one-level FP64 solves: the FP32 ones also want (r, r) and the column sums of the update
+template <typename T>
+static inline bool update_level(const GridDev &g, int precond) {
+    return std::is_same<T, double>::value && g.nz == 1 && precond == 2;
+}
+
 // An update of more workgroups than this takes its scalars from one workgroup launched before
-// it: every workgroup of the update would wait for the records again (515 x 515 columns at
-// nz = 1, 4,145 workgroups: 190 ms a solve against 201; 163 x 163 x 21, 415: 518 against 523)
-#define CG_FUSE_BLOCKS 1024
+// it: every workgroup of the update would wait for the records again.  515 x 515 columns at
+// nz = 1 with 4,145 workgroups (64 columns each): 190 ms a solve against 201 ms adding them
+// itself; with 1,036 (256 columns each): 138 against 136; 163 x 163 x 21, 415: 523 against 518.
+#define CG_FUSE_BLOCKS 2048
 static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop) {
     const RedSrc src = red_source<2>(c, part, nb);
     if (nblk <= CG_FUSE_BLOCKS) return src;
@@ -1264,7 +1300,10 @@ static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, const RedSrc
             if (precond == PRECOND_SIA_COARSE) cs = c->coarse->colsum;
         const int32_t *um = cs && c->dirichlet_any ? c->umask : nullptr;
         const int32_t *vm = cs && c->dirichlet_any ? c->vmask : nullptr;
-        if (g.nz <= 12)
+        if (update_level<T>(g, precond))
+            hipLaunchKernelGGL(k_cg_update_level<T>, dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0, c->stream, g, v.z,
+                               v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F);
+        else if (g.nz <= 12)
             hipLaunchKernelGGL((k_cg_update_sia<T, 12>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
                                v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
                                um, vm);
@@ -1307,7 +1346,8 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     // an inner solve (check = 1) whose residual becomes exactly zero has converged; the
     // reference recurrences would divide 0 by 0 there
     const int zero_stop = check;
-    const int nbu = precond >= 2 ? sia_blocks(g) : nbm;   // workgroups of the update
+    // workgroups of the update
+    const int nbu = precond < 2 || update_level<T>(g, precond) ? nbm : sia_blocks(g);
     int cur = 0;                // the CgState that holds the current scalars
     bool checked = false;       // the last launch was a convergence check
     hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, c->stream, c->sc);

@@ -1,6 +1,6 @@
 """The dot products that the PCG kernels add for themselves, at the sizes where their form
 changes: one record a group (up to 64 node blocks), up to eight (512), more (a launch of its
-own), and updates of more than 1024 workgroups, whose scalars come from one workgroup.  A dozen
+own), and updates of more than 2048 workgroups, whose scalars come from one workgroup.  A dozen
 iterations from the same start against the oracle, as in test_gpu_parity.test_pcg_short: only
 the order of the global sums differs, so the iterates agree to rounding (1e-11).  Twelve
 iterations end between two convergence checks, eleven leave a standard PCG's halo as it is."""
@@ -19,6 +19,7 @@ SIZES = {                                # nodes nz (ewn + 3) (nsn + 3) in block
     "512_blocks": (125, 125, 8),
     "513_blocks": (126, 125, 8),
     "1040_update_blocks": (254, 256, 2),
+    "2105_update_blocks": (364, 364, 2),
 }
 
 
