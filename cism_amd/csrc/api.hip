@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(256) void k_noslip_masks(GridDev g, int noslip, int
                                                       int32_t *__restrict__ vm) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int m = noslip && (int)(q % g.nz) == g.nz - 1;
+    const int m = noslip && node_level(g, q) == g.nz - 1;
     um[q] = m;
     vm[q] = m;
 }

@@ -550,7 +550,7 @@ __global__ __launch_bounds__(256) void k_gather(GridDev g, const int32_t *__rest
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q < (int)g.nn) {
     const int k = q % g.nz + 1;                // 1-based
-    const int col = q / g.nz;
+    const int col = node_col(g, q);
     const int i = col % g.sx + 1, j = col / g.sx + 1;
     const int nzm = g.nz - 1;
     // candidate elements: cell (i+dI, j+dJ), layer k-1+dK
@@ -698,7 +698,7 @@ __global__ __launch_bounds__(256) void k_basal_standard(GridDev g, const int32_t
     const int s = (int)(t / ncol);
     const long long col = t - s * ncol;
     const int iA = s % 3 - 1, jA = s / 3 - 1;
-    const int ii = (int)(col % g.sx) + 1, jj = (int)(col / g.sx) + 1;   // 1-based vertex
+    const int ii = col_i(g, col) + 1, jj = col_j(g, col) + 1;   // 1-based vertex
     // corners SW, SE, NE, NW of a cell relative to its NE vertex (ishift(3, n), jshift(3, n))
     const int di[4] = {-1, 0, 0, -1}, dj[4] = {-1, -1, 0, 0};
     const double r3 = 1.0 / sqrt(3.0);
@@ -831,9 +831,9 @@ __global__ __launch_bounds__(256) void k_dirichlet(GridDev g, const int32_t *__r
                                                    double *__restrict__ A, double *__restrict__ b) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz) + 1;
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx) + 1, j = (int)(col / g.sx) + 1;
+    const int k = node_level(g, q) + 1;
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col) + 1, j = col_j(g, col) + 1;
     // prescribed-node loop range: i, j in nhalo .. n-nhalo+1 and active (velo_higher:8441-8443)
     auto in_range = [&](int ii, int jj) {
         return ii >= CISM_NHALO && ii <= g.nx - CISM_NHALO + 1 && jj >= CISM_NHALO &&
@@ -947,10 +947,10 @@ __global__ __launch_bounds__(256) void k_sym_repair(GridDev g, const int32_t *__
     int k = 0, i = 0, j = 0;
     long long col = 0;
     if (!skip) {
-        k = (int)(q % g.nz);
-        col = q / g.nz;
-        i = (int)(col % g.sx);
-        j = (int)(col / g.sx);
+        k = node_level(g, q);
+        col = node_col(g, q);
+        i = col_i(g, col);
+        j = col_j(g, col);
         skip = ac && !av[col] && !av_prev[col] && is_owned(g, i, j) && !touches_active_cell(g, ac, i, j) &&
                !touches_active_cell(g, ac_prev, i, j);
     }
@@ -1096,8 +1096,8 @@ __global__ __launch_bounds__(256) void k_nnz(GridDev g, const int32_t *__restric
                                              const double *__restrict__ A, double *__restrict__ partials) {
     double acc[1] = {0.0};
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col), j = col_j(g, col);
     if (q < g.nn && is_owned(g, i, j) && av[col]) {
         int n = 0;
         for (int m = 0; m < 27; ++m) {
@@ -1136,9 +1136,9 @@ __global__ __launch_bounds__(256) void k_resvec(GridDev g, const int32_t *__rest
     // one lane per node
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q < g.nn) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const int k = node_level(g, q);
+        const long long col = node_col(g, q);
+        int i = col_i(g, col), j = col_j(g, col);
         const bool own = is_owned(g, i, j);
         long long qs = q;     // row whose product this lane forms
         bool none = false;    // a halo row without an image
@@ -1151,7 +1151,7 @@ __global__ __launch_bounds__(256) void k_resvec(GridDev g, const int32_t *__rest
         }
         double ru = 0.0, rv = 0.0;
         bool act = false;
-        if (!none && av[qs / g.nz]) {
+        if (!none && av[node_col(g, qs)]) {
             act = true;
             double su = 0.0, sv = 0.0;
 #pragma unroll
@@ -1216,9 +1216,9 @@ __global__ __launch_bounds__(256) void k_resvel(GridDev g, int whichresid, const
     const long long stride = (long long)gridDim.x * blockDim.x;
     const int kmax = (whichresid == 1 || whichresid == 2) ? g.nz - 1 : g.nz;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const int k = node_level(g, q);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         if (!is_owned(g, i, j) || k >= kmax) continue;
         const double u = x[2 * q], v = x[2 * q + 1];
         const double speed = sqrt(u * u + v * v);
@@ -1253,8 +1253,8 @@ __global__ __launch_bounds__(256) void k_load_local(GridDev g, const double *__r
                                                     double *__restrict__ load) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz) + 1;
-    const long long col = q / g.nz;
+    const int k = node_level(g, q) + 1;
+    const long long col = node_col(g, q);
     if (!av[col]) return;
     const double dz = sthck[col] * (wsig[k] - wsig[k - 1]);
     const double f = CISM_RHOI * CISM_GRAV * dx * dy * dz / CISM_VOL0;
@@ -1273,9 +1273,9 @@ __global__ __launch_bounds__(256) void k_load_standard(GridDev g, const double *
                                                        double *__restrict__ load) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz) + 1;
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx) + 1, j = (int)(col / g.sx) + 1;
+    const int k = node_level(g, q) + 1;
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col) + 1, j = col_j(g, col) + 1;
     double lu = load[2 * q], lv = load[2 * q + 1];
     const double r = 1.0 / sqrt(3.0);
     for (int dJ = 0; dJ < 2; ++dJ)
@@ -1362,9 +1362,9 @@ __global__ __launch_bounds__(256) void k_load_lateral(GridDev g, const double *_
                                                       double *__restrict__ load) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz) + 1;
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx) + 1, j = (int)(col / g.sx) + 1;
+    const int k = node_level(g, q) + 1;
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col) + 1, j = col_j(g, col) + 1;
     auto C2i = [&](const int32_t *a, int ii, int jj) { return a[(ii - 1) + (long long)g.nx * (jj - 1)]; };
     auto V2 = [&](const double *a, int ii, int jj) { return a[(ii - 1) + (long long)g.sx * (jj - 1)]; };
     double lu = load[2 * q], lv = load[2 * q + 1];

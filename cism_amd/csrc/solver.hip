@@ -129,30 +129,46 @@ struct RedSrc {
 };
 
 // The sums reach thread 0 only (after the barrier): 64 dependent additions by every lane
-// would cost a full CU more than the launches they replace.
+// would cost a full CU more than the launches they replace.  Lane c adds value c's groups, 16
+// of them read ahead of the additions (0.85 us of a 3 us kernel reading them one by one).
 template <int NV>
 __device__ __forceinline__ void red_sums(const RedSrc &src, double (&out)[NV]) {
-    __shared__ double grp[RED_GROUPS][NV];
+    alignas(16) __shared__ double grp[NV][RED_GROUPS];
     for (int t = threadIdx.x; t < RED_GROUPS * NV; t += blockDim.x) {
         const int c = t % NV, b0 = (t / NV) * src.chunk;
         double v[RED_CHUNK];
 #pragma unroll
-        for (int u = 0; u < RED_CHUNK; ++u)
-            v[u] = u < src.chunk && b0 + u < src.n ? src.p[(size_t)(b0 + u) * NV + c] : 0.0;
+        for (int u = 0; u < RED_CHUNK; ++u) {   // unconditional loads, record 0 for none
+            const bool in = u < src.chunk && b0 + u < src.n;
+            const double w = src.p[(size_t)(in ? b0 + u : 0) * NV + c];
+            v[u] = in ? w : 0.0;
+        }
 #pragma unroll
         for (int off = RED_CHUNK / 2; off > 0; off >>= 1)
 #pragma unroll
             for (int u = 0; u < off; ++u) v[u] += v[u + off];
-        grp[t / NV][c] = v[0];
+        grp[c][t / NV] = v[0];
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {   // one wave
+        const double2 *g2 = reinterpret_cast<const double2 *>(grp[threadIdx.x < NV ? threadIdx.x : 0]);
+        double s = 0.0;
 #pragma unroll
-        for (int c = 0; c < NV; ++c) out[c] = grp[0][c];
+        for (int h = 0; h < RED_GROUPS / 16; ++h) {
+            double2 v[8];
 #pragma unroll
-        for (int g = 1; g < RED_GROUPS; ++g)
+            for (int u = 0; u < 8; ++u) v[u] = g2[8 * h + u];
+            __builtin_amdgcn_sched_barrier(0);
+            s = h ? s + v[0].x : v[0].x;
+            s += v[0].y;
 #pragma unroll
-            for (int c = 0; c < NV; ++c) out[c] += grp[g][c];
+            for (int u = 1; u < 8; ++u) {
+                s += v[u].x;
+                s += v[u].y;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NV; ++c) out[c] = __shfl(s, c, 64);
     }
 }
 
@@ -407,9 +423,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_matvec(GridDev g, const T *__res
                                                        const T *__restrict__ x, T *__restrict__ y) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz);
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const int k = node_level(g, q);
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col), j = col_j(g, col);
     T yu = 0, yv = 0;
     if (is_owned(g, i, j) && av[col]) row_product<T>(g, MatFull<T>{A}, x, q, k, yu, yv);
     store2<T>(y, q, yu, yv);
@@ -439,9 +455,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, unsigned 
     if (M::xcd && lb * blockDim.x >= g.nn) return;
     const long long q = lb * blockDim.x + threadIdx.x;
     if (q < g.nn) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const int k = node_level(g, q);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         T yu = 0, yv = 0;
         const bool own = is_owned(g, i, j);
         if (own && av[col]) row_product<T>(g, A, x, q, k, yu, yv);
@@ -470,9 +486,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_residual(GridDev g, unsigned chu
     if (M::xcd && lb * blockDim.x >= g.nn) return;
     const long long q = lb * blockDim.x + threadIdx.x;
     if (q < g.nn) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const int k = node_level(g, q);
+        const long long col = node_col(g, q);
+        int i = col_i(g, col), j = col_j(g, col);
         const bool own = is_owned(g, i, j);
         long long qs = q;     // row whose value this entry takes
         bool zero = false;
@@ -484,7 +500,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_residual(GridDev g, unsigned chu
         T ru = 0, rv = 0;
         if (!zero) {
             T yu = 0, yv = 0;
-            const long long cs = qs / g.nz;
+            const long long cs = node_col(g, qs);
             if (is_owned(g, i, j) && av[cs]) row_product<T>(g, A, x, qs, k, yu, yv);
             ru = b[2 * qs] - yu;
             rv = b[2 * qs + 1] - yv;
@@ -503,8 +519,8 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_dot(GridDev g, const T *__restri
     double acc[1] = {0.0};
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         if (is_owned(g, i, j))
             acc[0] += (double)a[2 * q] * (double)b[2 * q] + (double)a[2 * q + 1] * (double)b[2 * q + 1];
     }
@@ -632,7 +648,7 @@ __global__ __launch_bounds__(128) void k_sia_setup_sym32(GridDev g, const float 
 
 // One column and component of the SIA preconditioner: the Thomas substitutions
 // on s (level k at s[2k]) with the factors precomputed by k_sia_setup.  For
-// nz <= 12 the factors are first loaded into registers (sia_factors), so that a
+// nz <= 24 the factors are first loaded into registers (sia_factors), so that a
 // caller can issue those loads early; the substitutions would otherwise wait on
 // one global load per level.
 template <typename T, int NZMAX>
@@ -676,7 +692,7 @@ __device__ __forceinline__ void sia_solve(int nz, const SiaFactors<T, NZMAX> &f,
 template <typename T, int NZMAX>
 __device__ __forceinline__ void sia_column(int nz, long long ncol, const T *__restrict__ F, long long col,
                                            int comp, T *s) {
-    if constexpr (NZMAX <= 12) {
+    if constexpr (NZMAX <= 24) {
         SiaFactors<T, NZMAX> f;
         sia_factors<T, NZMAX>(nz, ncol, F, col, comp, f);
         sia_solve<T, NZMAX>(nz, f, s);
@@ -722,7 +738,7 @@ __global__ __launch_bounds__(128) void k_sia_apply(GridDev g, const T *__restric
     const long long col = col0 + lc;
     if (lc < ncols && av[col]) {
         if (colsum) {
-            const int jc = (int)(col / g.sx), ic = (int)(col - (long long)jc * g.sx);
+            const int jc = col_j(g, col), ic = (int)(col - (long long)jc * g.sx);
             if (is_owned(g, ic, jc)) {
                 const int32_t *dm = comp == 0 ? um : vm;
                 T cs = (T)0;
@@ -818,8 +834,8 @@ static int launch_precond(cism_ctx *c, int precond, const M A, const T *F, const
 __device__ inline bool halo_vertex_of(const GridDev &g, long long h, int &i, int &j) {
     const long long nrow = 3LL * g.sx;
     if (h < nrow) {
-        const int rr = (int)(h / g.sx);
-        i = (int)(h % g.sx);
+        const int rr = col_j(g, h);
+        i = col_i(g, h);
         j = rr < 2 ? rr : g.sy - 1;
         return true;
     }
@@ -840,11 +856,11 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_halo(GridDev g, T *__restrict__ 
     const int NV = MAT ? 108 : 2;
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nh * NV) return;
-    const int p = (int)(t / nh);           // value index (block*27+slot, or component)
-    const long long hv = t % nh;
-    const int k = (int)(hv % g.nz);
+    const int p = MAT ? (int)(t / nh) : t >= nh;   // value index (block*27+slot, or component)
+    const long long hv = t - p * nh;
+    const int k = node_level(g, hv);
     int i, j;
-    if (!halo_vertex_of(g, hv / g.nz, i, j)) return;
+    if (!halo_vertex_of(g, node_col(g, hv), i, j)) return;
     const int ii = halo_image(i, g.sx, g.periodic), jj = halo_image(j, g.sy, g.periodic);
     const long long qd = k + (long long)g.nz * (i + (long long)g.sx * j);
     const long long qs = k + (long long)g.nz * (ii + (long long)g.sx * jj);
@@ -871,9 +887,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_a32_halo(GridDev g, float *__res
     if (t >= nh * CISM_SYM_SLOTS) return;
     const int s = (int)(t / nh);
     const long long hv = t % nh;
-    const int k = (int)(hv % g.nz);
+    const int k = node_level(g, hv);
     int i, j;
-    if (!halo_vertex_of(g, hv / g.nz, i, j)) return;
+    if (!halo_vertex_of(g, node_col(g, hv), i, j)) return;
     const int ii = halo_image(i, g.sx, g.periodic), jj = halo_image(j, g.sy, g.periodic);
     const long long q = k + (long long)g.nz * (i + (long long)g.sx * j);
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -947,9 +963,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned c
     double acc[1] = {0.0};
     const long long q = lb * blockDim.x + threadIdx.x;
     if (q < g.nn) {
-        const int k = (int)(q % g.nz);
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const int k = node_level(g, q);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         // the first node of the image of a column, or -1
         auto image = [&](int ii, int jj) {
             const int im = halo_image(ii, g.sx, g.periodic), jm = halo_image(jj, g.sy, g.periodic);
@@ -1044,7 +1060,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_update(GridDev g, const M A,
         if (precond <= 1) {
             const V2 zz = point_precond<T>(g, A, precond, q, rr);
             reinterpret_cast<V2 *>(z)[q] = zz;
-            const int col = (int)(q / g.nz), j = col / g.sx, i = col - j * g.sx;
+            const int col = node_col(g, q), j = col / g.sx, i = col - j * g.sx;
             if (is_owned(g, i, j)) acc[0] += (double)rr.x * (double)zz.x + (double)rr.y * (double)zz.y;
         }
     }
@@ -1053,62 +1069,74 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_update(GridDev g, const M A,
 
 // Chron-Gear (pcg:1517-1536) of node q with the halo update of Az (pcg:1494-1497)
 // folded in: halo entries read Az at their periodic image (or 0, outflow).
-// Returns 0 for a skipped node, 1 for an updated halo node, 2 for an updated owned one.
 //
 // skip_av (diagonal or SIA preconditioner only): owned nodes of inactive columns are
 // left alone.  There z = 0 (zeroed at the start, never written by those
 // preconditioners), A z = 0 and d = q = 0, so their update would rewrite d = q = 0
 // and leave x and r unchanged: skipping it changes no value and saves the traffic.
+//
+// In two parts, so that a kernel can have the loads under way while it waits for the scalars.
 template <typename T>
-__device__ __forceinline__ int cg_update_node(const GridDev &g, long long q, int k, long long col, int i,
-                                               int j, const T *__restrict__ z, const T *__restrict__ Az,
-                                               T *__restrict__ d, T *__restrict__ qv, T *__restrict__ x,
-                                               T *__restrict__ r, T alpha, T beta, int first,
-                                               const int32_t *__restrict__ skip_av,
-                                               typename Vec2<T>::t &rr) {
+struct CgNode {
+    typename Vec2<T>::t az, zz, d0, q0, xx, rr;
+    int state;   // 0 skipped, 1 halo, 2 owned
+};
+
+template <typename T>
+__device__ __forceinline__ void cg_load_node(const GridDev &g, long long q, int k, long long col, int i, int j,
+                                              const T *__restrict__ z, const T *__restrict__ Az,
+                                              const T *__restrict__ d, const T *__restrict__ qv,
+                                              const T *__restrict__ x, const T *__restrict__ r, int first,
+                                              const int32_t *__restrict__ skip_av, CgNode<T> &n) {
     // one lane per node (k, i, j) of column col: both components through one 8- or
     // 16-byte access per vector
     using V2 = typename Vec2<T>::t;
-    V2 az;
-    bool own;
-    {
-        own = is_owned(g, i, j);
-        if (own && skip_av && !skip_av[col]) return 0;
-        if (own) {
-            az = reinterpret_cast<const V2 *>(Az)[q];
-        } else {
-            const int ii = halo_image(i, g.sx, g.periodic), jj = halo_image(j, g.sy, g.periodic);
-            if (ii < 0 || jj < 0) {
-                az.x = (T)0;
-                az.y = (T)0;
-            } else {
-                az = reinterpret_cast<const V2 *>(Az)[k + (long long)g.nz * (ii + (long long)g.sx * jj)];
-            }
-        }
+    const bool own = is_owned(g, i, j);
+    n.state = own ? 2 : 1;
+    if (own && skip_av && !skip_av[col]) {
+        n.state = 0;
+        return;
     }
-    const V2 zz = reinterpret_cast<const V2 *>(z)[q];
+    n.az.x = n.az.y = (T)0;
+    if (own) {
+        n.az = reinterpret_cast<const V2 *>(Az)[q];
+    } else {
+        const int ii = halo_image(i, g.sx, g.periodic), jj = halo_image(j, g.sy, g.periodic);
+        if (ii >= 0 && jj >= 0)
+            n.az = reinterpret_cast<const V2 *>(Az)[k + (long long)g.nz * (ii + (long long)g.sx * jj)];
+    }
+    n.zz = reinterpret_cast<const V2 *>(z)[q];
+    if (!first) {
+        n.d0 = reinterpret_cast<const V2 *>(d)[q];
+        n.q0 = reinterpret_cast<const V2 *>(qv)[q];
+    }
+    n.xx = reinterpret_cast<const V2 *>(x)[q];
+    n.rr = reinterpret_cast<const V2 *>(r)[q];
+}
+
+// n.rr becomes the new r
+template <typename T>
+__device__ __forceinline__ void cg_apply_node(long long q, T *__restrict__ d, T *__restrict__ qv, T *__restrict__ x,
+                                               T *__restrict__ r, T alpha, T beta, int first, CgNode<T> &n) {
+    using V2 = typename Vec2<T>::t;
     V2 dd, qq;
     if (first) {   // first pass: d = z, q = A d (already halo-mapped), pcg:1351-1405
-        dd = zz;
-        qq = az;
+        dd = n.zz;
+        qq = n.az;
     } else {
-        const V2 d0 = reinterpret_cast<const V2 *>(d)[q], q0 = reinterpret_cast<const V2 *>(qv)[q];
-        dd.x = zz.x + beta * d0.x;
-        dd.y = zz.y + beta * d0.y;
-        qq.x = az.x + beta * q0.x;
-        qq.y = az.y + beta * q0.y;
+        dd.x = n.zz.x + beta * n.d0.x;
+        dd.y = n.zz.y + beta * n.d0.y;
+        qq.x = n.az.x + beta * n.q0.x;
+        qq.y = n.az.y + beta * n.q0.y;
     }
     reinterpret_cast<V2 *>(d)[q] = dd;
     reinterpret_cast<V2 *>(qv)[q] = qq;
-    V2 xx = reinterpret_cast<const V2 *>(x)[q];
-    rr = reinterpret_cast<const V2 *>(r)[q];
-    xx.x = xx.x + alpha * dd.x;
-    xx.y = xx.y + alpha * dd.y;
-    rr.x = rr.x - alpha * qq.x;
-    rr.y = rr.y - alpha * qq.y;
-    reinterpret_cast<V2 *>(x)[q] = xx;
-    reinterpret_cast<V2 *>(r)[q] = rr;
-    return own ? 2 : 1;
+    n.xx.x = n.xx.x + alpha * dd.x;
+    n.xx.y = n.xx.y + alpha * dd.y;
+    n.rr.x = n.rr.x - alpha * qq.x;
+    n.rr.y = n.rr.y - alpha * qq.y;
+    reinterpret_cast<V2 *>(x)[q] = n.xx;
+    reinterpret_cast<V2 *>(r)[q] = n.rr;
 }
 
 template <typename T>
@@ -1119,15 +1147,17 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update(GridDev g, const T *__
                                                           DevScal *__restrict__ sc, int cur, int first,
                                                           int zero_stop,
                                                           const int32_t *__restrict__ skip_av) {
+    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    CgNode<T> n;
+    n.state = 0;
+    if (q < g.nn) {
+        const int col = node_col(g, q);
+        cg_load_node<T>(g, q, node_level(g, q), col, col_i(g, col), col_j(g, col), z, Az, d, qv, x, r, first, skip_av,
+                        n);
+    }
     double alpha, beta;
     cg_scalars(src, sc, cur, first, zero_stop, alpha, beta);
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= g.nn) return;
-    const int k = (int)(q % g.nz);
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
-    typename Vec2<T>::t rr;
-    cg_update_node<T>(g, q, k, col, i, j, z, Az, d, qv, x, r, (T)alpha, (T)beta, first, skip_av, rr);
+    if (n.state) cg_apply_node<T>(q, d, qv, x, r, (T)alpha, (T)beta, first, n);
 }
 
 // The Chron-Gear update followed by the SIA preconditioner of the next iteration
@@ -1140,7 +1170,11 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update(GridDev g, const T *__
 // convergence check of the inner solves, pcg:1540-1560).  With colsum the block also
 // leaves the (u, v) sums of the new r over the levels of its owned active columns, the
 // first stage of the coarse correction's restriction (coarse.hip).
-template <typename T, int NZMAX>
+//
+// FUSED: the workgroup forms the scalars itself, with its first node's vectors under way.  Without
+// it (many workgroups, k_cg_scalars before) the kernel keeps to 68 registers at FP32 and 12
+// levels instead of 97: 551 ms a 1200 x 1400 x 11 solve, 563 with them.
+template <typename T, int NZMAX, bool FUSED>
 __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T *__restrict__ Az,
                                                        T *__restrict__ d, T *__restrict__ qv,
                                                        T *__restrict__ x, T *__restrict__ r, RedSrc src,
@@ -1161,33 +1195,40 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
     const int comp = (threadIdx.x >> 6) & 1, lc = threadIdx.x & 63;
     const long long col = col0 + lc;
     const bool solve = threadIdx.x < 128 && lc < ncols && av[col];
-    SiaFactors<T, (NZMAX <= 12 ? NZMAX : 1)> f;
-    if constexpr (NZMAX <= 12)
+    SiaFactors<T, (NZMAX <= 24 ? NZMAX : 1)> f;
+    if constexpr (NZMAX <= 24)
         if (solve) sia_factors<T, NZMAX>(nz, ncol, F, col, comp, f);
+    // node t of the block: level t % nz of local column t / nz (32-bit: the context
+    // limits grids to 2^30 nodes).
+    const int c0 = (int)col0;
+    auto load = [&](int t, CgNode<T> &n) {
+        const int lcol = (int)((unsigned)t / (unsigned)nz), cn = c0 + lcol, jn = col_j(g, cn);
+        cg_load_node<T>(g, Q0 + t, t - lcol * nz, cn, cn - jn * g.sx, jn, z, Az, d, qv, x, r, first, av, n);
+    };
+    CgNode<T> n;
     double alpha64, beta64;
-    cg_scalars(src, sc, cur, first, zero_stop, alpha64, beta64);
+    if constexpr (FUSED) {
+        if ((int)threadIdx.x < nn) load(threadIdx.x, n);
+        cg_scalars(src, sc, cur, first, zero_stop, alpha64, beta64);
+    } else {
+        alpha64 = sc->cg[cur ^ 1].alpha;
+        beta64 = sc->cg[cur ^ 1].beta;
+    }
     const T alpha = (T)alpha64, beta = (T)beta64;
     double acc[1] = {0.0};
-    // node t of the block: level t % nz of local column t / nz (32-bit: the context
-    // limits grids to 2^30 nodes)
-    const int c0 = (int)col0;
     for (int t = threadIdx.x; t < nn; t += blockDim.x) {
-        const int lcol = t / nz;
-        const int cn = c0 + lcol;
-        const int jn = cn / g.sx;
-        typename Vec2<T>::t rr;
-        const int st = cg_update_node<T>(g, Q0 + t, t - lcol * nz, cn, cn - jn * g.sx, jn, z, Az, d, qv, x, r,
-                                         alpha, beta, first, av, rr);
-        if (st) {
-            sr[2 * t] = rr.x;
-            sr[2 * t + 1] = rr.y;
-            if (st == 2) acc[0] += (double)rr.x * rr.x + (double)rr.y * rr.y;
+        if (!FUSED || t >= (int)blockDim.x) load(t, n);
+        if (n.state) {
+            cg_apply_node<T>(Q0 + t, d, qv, x, r, alpha, beta, first, n);
+            sr[2 * t] = n.rr.x;
+            sr[2 * t + 1] = n.rr.y;
+            if (n.state == 2) acc[0] += (double)n.rr.x * n.rr.x + (double)n.rr.y * n.rr.y;
         }
     }
     __syncthreads();
     if (solve) {
         if (colsum) {
-            const int jc = (int)(col / g.sx), ic = (int)(col - (long long)jc * g.sx);
+            const int jc = col_j(g, col), ic = (int)(col - (long long)jc * g.sx);
             if (is_owned(g, ic, jc)) {
                 // prescribed (Dirichlet) components stay out of the coarse space
                 const int32_t *dm = comp == 0 ? um : vm;
@@ -1197,7 +1238,7 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
                 colsum[2 * col + comp] = cs;
             }
         }
-        if constexpr (NZMAX <= 12) sia_solve<T, NZMAX>(nz, f, sr + 2 * lc * nz + comp);
+        if constexpr (NZMAX <= 24) sia_solve<T, NZMAX>(nz, f, sr + 2 * lc * nz + comp);
         else sia_column<T, NZMAX>(nz, ncol, F, col, comp, sr + 2 * lc * nz + comp);
     }
     __syncthreads();
@@ -1226,13 +1267,15 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update_level(GridDev g, T *z,
         bu = F[2 * ncol + q];
         bv = F[3 * ncol + q];
     }
+    CgNode<T> n;
+    n.state = 0;
+    if (q < ncol) cg_load_node<T>(g, q, 0, q, col_i(g, q), col_j(g, q), z, Az, d, qv, x, r, first, av, n);
     double alpha, beta;
     cg_scalars(src, sc, cur, first, zero_stop, alpha, beta);
-    if (q >= ncol) return;
-    const int j = (int)(q / g.sx), i = (int)(q - (long long)j * g.sx);
-    V2 rr;
-    const int st = cg_update_node<T>(g, q, 0, q, i, j, z, Az, d, qv, x, r, (T)alpha, (T)beta, first, av, rr);
-    if (st && solve) store2<T>(z, q, rr.x / bu, rr.y / bv);
+    if (n.state) {
+        cg_apply_node<T>(q, d, qv, x, r, (T)alpha, (T)beta, first, n);
+        if (solve) store2<T>(z, q, n.rr.x / bu, n.rr.y / bv);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1303,18 +1346,13 @@ static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, const RedSrc
         if (update_level<T>(g, precond))
             hipLaunchKernelGGL(k_cg_update_level<T>, dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0, c->stream, g, v.z,
                                v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F);
-        else if (g.nz <= 12)
-            hipLaunchKernelGGL((k_cg_update_sia<T, 12>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
-                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
-                               um, vm);
-        else if (g.nz <= 24)
-            hipLaunchKernelGGL((k_cg_update_sia<T, 24>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
-                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
-                               um, vm);
-        else
-            hipLaunchKernelGGL((k_cg_update_sia<T, 48>), grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q,
-                               v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F, want_rr, c->partials, cs,
-                               um, vm);
+        else {
+            auto kern = g.nz <= 12   ? (src.n ? k_cg_update_sia<T, 12, true> : k_cg_update_sia<T, 12, false>)
+                        : g.nz <= 24 ? (src.n ? k_cg_update_sia<T, 24, true> : k_cg_update_sia<T, 24, false>)
+                                     : (src.n ? k_cg_update_sia<T, 48, true> : k_cg_update_sia<T, 48, false>);
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, c->stream, g, v.z, v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur,
+                               first, zero_stop, c->av, v.F, want_rr, c->partials, cs, um, vm);
+        }
         HIP_TRY(hipGetLastError());
         if constexpr (std::is_same<T, float>::value)
             if (precond == PRECOND_SIA_COARSE) CISM_TRY(coarse_apply(c, v.z));
@@ -1538,8 +1576,8 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_rhs32(GridDev g, long long n2, c
         z32[q] = 0.0f;
         const long long node = q >> 1;
         if (node < g.nn) {
-            const long long col = node / g.nz;
-            if (is_owned(g, (int)(col % g.sx), (int)(col / g.sx))) acc[0] = (double)v * v;
+            const long long col = node_col(g, node);
+            if (is_owned(g, col_i(g, col), col_j(g, col))) acc[0] = (double)v * v;
         }
     }
     block_reduce_store<1>(acc, partials);
@@ -1680,7 +1718,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_colscale(GridDev g, const double
     if (t >= 2 * ncol) return;
     const int comp = (int)(t / ncol);
     const long long col = t - comp * ncol;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const int i = col_i(g, col), j = col_j(g, col);
     double s = 1.0;
     if (is_owned(g, i, j) && av[col]) {
         const int blk = comp == 0 ? 0 : 3;
@@ -1712,8 +1750,8 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_energy(GridDev g, const int32_t 
     double acc[2] = {0.0, 0.0};
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         if (is_owned(g, i, j) && av[col]) {
             acc[0] += x[2 * q] * t[2 * q] + x[2 * q + 1] * t[2 * q + 1];
             acc[1] += b[2 * q] * x[2 * q] + b[2 * q + 1] * x[2 * q + 1];
@@ -1763,8 +1801,8 @@ int column_scale_device(cism_ctx *c, double *out) {
 __device__ inline bool aa_entry_active(const GridDev &g, const int32_t *__restrict__ av, long long t) {
     const long long q = t >> 1;
     if (q >= g.nn) return false;
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col), j = col_j(g, col);
     return is_owned(g, i, j) && av[col];
 }
 
@@ -1798,8 +1836,8 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_aa_dots(GridDev g, const int32_t
     for (int c = 0; c < AA_NV; ++c) acc[c] = 0.0;
     const long long gs = (long long)gridDim.x * blockDim.x;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += gs) {
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         if (!is_owned(g, i, j) || !av[col]) continue;
         double2 v2[AA_MAX];
 #pragma unroll
@@ -1978,7 +2016,7 @@ int launch_cg_matvec(cism_ctx *c, int which) {
 // inner solves issue it (vectors, factors and scalars of the last mixed solve)
 int launch_cg_update32(cism_ctx *c) {
     CGVecs<float> v = {c->x32, c->b32, c->r32, c->d32, c->z32, c->q32, c->Az32, c->F32, nullptr};
-    const RedSrc src = {c->red_groups, RED_GROUPS, 1};
+    const RedSrc src = {nullptr, 0, 0};   // the scalars of the last iteration
     return launch_cg_update<float>(c, 2, v, src, 0, 0, 1, 1);
 }
 
@@ -1989,8 +2027,8 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_err_sums(GridDev g, const double
     double acc[2] = {0.0, 0.0};
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g.nn; q += stride) {
-        const long long col = q / g.nz;
-        const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+        const long long col = node_col(g, q);
+        const int i = col_i(g, col), j = col_j(g, col);
         if (!is_owned(g, i, j)) continue;
         const double du = x[2 * q] - xr[2 * q], dv = x[2 * q + 1] - xr[2 * q + 1];
         acc[0] += du * du + dv * dv;

@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256) void k_gather_2d(GridDev g, const int32_t *__r
                                                    double basal_scale, double *__restrict__ A) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // vertex = node
     if (q >= (long long)g.sx * g.sy) return;
-    const int iv = (int)(q % g.sx) + 1, jv = (int)(q / g.sx) + 1;
+    const int iv = col_i(g, q) + 1, jv = col_j(g, q) + 1;
     long long cid[4];
     bool cv[4];
     int nr[4];
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(256) void k_beta_eff(GridDev g, const double *__res
                                                   int noslip, double *__restrict__ som, double *__restrict__ beff) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (long long)g.sx * g.sy) return;
-    const int i = (int)(q % g.sx), j = (int)(q / g.sx);
+    const int i = col_i(g, q), j = col_j(g, q);
     const double s = stagger_m1(g.nx, om, ipl, i, j);
     som[q] = s;
     if (noslip) beff[q] = s > 0.0 ? 1.0 / s : 0.0;
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) void k_diva_velocity(GridDev g, int nz3, const
     if (t >= ncol * nz3) return;
     const long long q = t / nz3;
     const int k = (int)(t - q * nz3);
-    const int i = (int)(q % g.sx), j = (int)(q / g.sx);
+    const int i = col_i(g, q), j = col_j(g, q);
     const double u2 = vel[2 * q], v2 = vel[2 * q + 1];
     const double tx = beff[q] * u2, ty = beff[q] * v2;
     if (k == nz3 - 1) {
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256) void k_halo_lead(GridDev g, int lead, double *
     if (t >= ncol * lead) return;
     const int k = (int)(t % lead);
     const long long q = t / lead;
-    const int i = (int)(q % g.sx), j = (int)(q / g.sx);
+    const int i = col_i(g, q), j = col_j(g, q);
     const int ii = halo_image(i, g.sx, g.periodic), jj = halo_image(j, g.sy, g.periodic);
     if (ii == i && jj == j) return;
     a[t] = (ii < 0 || jj < 0) ? 0.0 : a[k + (long long)lead * (ii + (long long)g.sx * jj)];
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(256) void k_zero_inactive(GridDev g, int nz3, const
                                                        double *__restrict__ v3) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= (long long)g.sx * g.sy) return;
-    const int i = (int)(q % g.sx), j = (int)(q / g.sx);
+    const int i = col_i(g, q), j = col_j(g, q);
     if (!is_owned(g, i, j) || av[q]) return;
     vel[2 * q] = 0.0;
     vel[2 * q + 1] = 0.0;
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256) void k_l1l2_column(GridDev g, DepthDev d, cons
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long ncol = (long long)g.sx * g.sy, ncell = (long long)g.nx * g.ny;
     if (q >= ncol) return;
-    const int i = (int)(q % g.sx), j = (int)(q / g.sx);
+    const int i = col_i(g, q), j = col_j(g, q);
     const int nz3 = d.nz3, L = nz3 - 1;
     double *uc = u3 + (long long)nz3 * q, *vc = v3 + (long long)nz3 * q;
     if (!is_owned(g, i, j) || !av[q]) {

@@ -1034,9 +1034,9 @@ __global__ __launch_bounds__(256) void k_guess_decode(GridDev g, int W, int Wown
                                                       const float *__restrict__ out, double *__restrict__ x) {
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.nn) return;
-    const int k = (int)(q % g.nz);
-    const long long col = q / g.nz;
-    const int i = (int)(col % g.sx), j = (int)(col / g.sx);
+    const int k = node_level(g, q);
+    const long long col = node_col(g, q);
+    const int i = col_i(g, col), j = col_j(g, col);
     const int px = i - i0, py = j - j0;
     double u = 0.0, v = 0.0;
     if (px >= 0 && px < Wown && py >= 0 && py < Hown && av[col]) {
