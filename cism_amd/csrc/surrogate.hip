@@ -102,9 +102,11 @@ __device__ __forceinline__ bool patch_pixel(const ConvDims &d, int off, int y0, 
 // mask (the data gradient of an input that went through a ReLU): zero where mask is not
 // positive.
 // Bound: the MFMA operands' L1 and LDS reads (2 + 2 KB per 4 MFMAs of a wave) at the deep
-// levels, the FP32 activations' traffic at the full resolution.  The twelve layers at 512 x 512:
-// 0.64 ms with every tap loaded and converted again and the concatenations written out,
-// 0.27 ms here.
+// levels, the FP32 activations' traffic at the full resolution.  The weights of four steps
+// are loaded ahead of the four being multiplied: waiting for each step's from L2 cost 6 to
+// 20% of a layer.  The twelve layers at 512 x 512: 0.64 ms with every tap loaded and converted
+// again and the concatenations written out, 0.29 ms with the patches and each step's weights
+// loaded as they were needed, 0.25 ms here.
 template <int NA>
 __global__ __launch_bounds__(256) void k_conv_patch(ConvDims d, ConvSrc src, const short *__restrict__ Wf,
                                                     const float *__restrict__ bias, const float *__restrict__ mask,
@@ -153,28 +155,44 @@ __global__ __launch_bounds__(256) void k_conv_patch(ConvDims d, ConvSrc src, con
         ci -= d.Ci;
         tap = 1;
     }
-#pragma unroll 4
-    for (int s = 0; s < S; ++s) {
-        bf16x8 af[NA], b0, b1;
+    // four steps' weights at a time, the next four on their way while these are multiplied
+    bf16x8 w0[4][NA], w1[4][NA];
+    auto weights = [&](bf16x8(&w)[4][NA], int s0) {
 #pragma unroll
-        for (int a = 0; a < NA; ++a) af[a] = wf[((long long)a * S + s) * 64];
-        const int ky = tap / 3, o = (ky * R + tap - 3 * ky) * ld + ci;
-        if (tap < d.ks * d.ks) {
-            b0 = *reinterpret_cast<const bf16x8 *>(xb0 + o);
-            b1 = *reinterpret_cast<const bf16x8 *>(xb1 + o);
-        } else {
-            b0 = b1 = bf16x8{};
-        }
+        for (int u = 0; u < 4; ++u)
+            if (s0 + u < S)
 #pragma unroll
-        for (int a = 0; a < NA; ++a) {
-            acc[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], b0, acc[a][0], 0, 0, 0);
-            acc[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], b1, acc[a][1], 0, 0, 0);
+                for (int a = 0; a < NA; ++a) w[u][a] = wf[((long long)a * S + s0 + u) * 64];
+    };
+    auto multiply = [&](const bf16x8(&w)[4][NA], int s0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (s0 + u >= S) break;
+            bf16x8 b0 = {}, b1 = {};
+            if (tap < d.ks * d.ks) {
+                const int ky = tap / 3, o = (ky * R + tap - 3 * ky) * ld + ci;
+                b0 = *reinterpret_cast<const bf16x8 *>(xb0 + o);
+                b1 = *reinterpret_cast<const bf16x8 *>(xb1 + o);
+            }
+#pragma unroll
+            for (int a = 0; a < NA; ++a) {
+                acc[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][a], b0, acc[a][0], 0, 0, 0);
+                acc[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][a], b1, acc[a][1], 0, 0, 0);
+            }
+            ci += 32;
+            if (ci >= d.Ci) {   // the next tap, or the one after it (16 channels)
+                const int over = d.Ci == 16 ? 2 : 1;
+                ci -= over * d.Ci;
+                tap += over;
+            }
         }
-        ci += 32;
-        while (ci >= d.Ci) {
-            ci -= d.Ci;
-            ++tap;
-        }
+    };
+    weights(w0, 0);
+    for (int s = 0; s < S; s += 8) {
+        weights(w1, s + 4);
+        multiply(w0, s);
+        weights(w0, s + 8);
+        multiply(w1, s + 4);
     }
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
