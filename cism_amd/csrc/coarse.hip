@@ -435,6 +435,21 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_restrict1(GridDev g, const in
     }
 }
 
+// r -= (A_l x)[c] for aggregate c = (ci, cj), its nine blocks in Ab, x(nb) the vector
+template <class X>
+__device__ __forceinline__ void cg_sub_row(int ci, int cj, int ax, int ay, int periodic, const float4 *Ab, X x,
+                                           float2 &r) {
+#pragma unroll
+    for (int d = 0; d < 9; ++d) {
+        const int nb = cg_nb(ci, cj, ax, ay, d % 3 - 1, d / 3 - 1, periodic);
+        if (nb < 0) continue;
+        const float4 B = Ab[d];
+        const float2 xn = x(nb);
+        r.x -= B.x * xn.x + B.y * xn.y;
+        r.y -= B.z * xn.x + B.w * xn.y;
+    }
+}
+
 // restriction of the pre-smoothed residual: r_{l+1}[P] = sum over children c of
 // (r_l - A_l e_l)[c]; with smooth, e_{l+1} = D_l1^-1 r_{l+1}
 __global__ __launch_bounds__(CISM_BLOCK) void k_cg_down(int axc, int ayc, int axp, int ayp, int periodic,
@@ -446,43 +461,22 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_down(int axc, int ayc, int ax
     const long long P = t >> 4;
     const int sub = (int)(t & 15);
     const bool okP = P < (long long)axp * ayp;
-    float ru = 0.0f, rv = 0.0f;
+    float2 rr = make_float2(0.0f, 0.0f);
     if (okP) {
         const int ci = CG_AGG * (int)(P % axp) + (sub & 3), cj = CG_AGG * (int)(P / axp) + (sub >> 2);
         if (ci < axc && cj < ayc) {
             const long long c = ci + (long long)axc * cj;
             const float2 *e2 = reinterpret_cast<const float2 *>(ec);
-            const float2 rr = reinterpret_cast<const float2 *>(rc)[c];
-            ru = rr.x;
-            rv = rr.y;
-            const float4 *Ab = reinterpret_cast<const float4 *>(A + c * 36);
-#pragma unroll
-            for (int d = 0; d < 9; ++d) {
-                const int nb = cg_nb(ci, cj, axc, ayc, d % 3 - 1, d / 3 - 1, periodic);
-                if (nb < 0) continue;
-                const float4 B = Ab[d];
-                const float2 en = e2[nb];
-                ru -= B.x * en.x + B.y * en.y;
-                rv -= B.z * en.x + B.w * en.y;
-            }
+            rr = reinterpret_cast<const float2 *>(rc)[c];
+            cg_sub_row(ci, cj, axc, ayc, periodic, reinterpret_cast<const float4 *>(A + c * 36),
+                       [&](int nb) { return e2[nb]; }, rr);
         }
     }
-    ru = cg_sum16(ru);
-    rv = cg_sum16(rv);
+    const float ru = cg_sum16(rr.x), rv = cg_sum16(rr.y);
     if (okP && sub == 0) {
         reinterpret_cast<float2 *>(rp)[P] = make_float2(ru, rv);
         if (smooth) reinterpret_cast<float2 *>(ep)[P] = make_float2(dl1p[2 * P] * ru, dl1p[2 * P + 1] * rv);
     }
-}
-
-// the coarsest level: e = Ainv r (one workgroup, n <= 2 CG_DENSE)
-__global__ __launch_bounds__(64) void k_cg_dense_apply(int n, const float *__restrict__ Ainv,
-                                                       const float *__restrict__ r, float *__restrict__ e) {
-    const int i = threadIdx.x;
-    if (i >= n) return;
-    float s = 0.0f;
-    for (int j = 0; j < n; ++j) s += Ainv[i * n + j] * r[j];
-    e[i] = s;
 }
 
 // prolongation and post-smoothing on level l: with e' = e_l + Q e_{l+1} (Q the parent
@@ -500,19 +494,123 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_up(int ax, int ay, int axp, i
         return make_float2(x.x + y.x, x.y + y.y);
     };
     const float2 ec = corr((int)c);
-    const float2 rr = reinterpret_cast<const float2 *>(r)[c];
-    float ru = rr.x, rv = rr.y;
-    const float4 *Ab = reinterpret_cast<const float4 *>(A + c * 36);
+    float2 rr = reinterpret_cast<const float2 *>(r)[c];
+    cg_sub_row(ci, cj, ax, ay, periodic, reinterpret_cast<const float4 *>(A + c * 36), corr, rr);
+    reinterpret_cast<float2 *>(eo)[c] = make_float2(ec.x + dl1[2 * c] * rr.x, ec.y + dl1[2 * c + 1] * rr.y);
+}
+
+// The V-cycle's coarse end in one workgroup: from r and the pre-smoothed e of its first level,
+// k_cg_down to the coarsest level, the dense inverse there, and k_cg_up back to the first
+// level's eo, with the same sums in the same order.  NL levels are smoothed; their coarse
+// vectors stay in LDS, and a lane keeps its child's nine blocks in registers from the way down
+// to the way up.  Its first level is the first whose children fit the workgroup, one lane each
+// (16 lanes per parent, at most CG_TAIL parents), so a level under it has at most CG_TAIL
+// aggregates and the one under that at most 16: NL <= 2.
+// Bound: one compute unit's load of the blocks (147 KB at 32 x 32 aggregates) and the latency
+// of its phases.  A 512 x 512 grid (32 x 32, 8 x 8, 2 x 2 under its first level): 24 us in five
+// launches and the gaps between them, 13 us here (the solve: -1.6%).  Blocks stored by
+// direction ([d][a]) make this 11.6 us and the first level's k_cg_down and k_cg_up, which
+// read a whole row per lane, 1.2 us slower each.
+#define CG_TAIL 64
+static_assert(CG_TAIL / CG_AGG <= CG_DENSE, "two levels above the coarsest");
+struct CgTail {
+    int periodic;
+    CoarseLevel lev[3];   // NL + 1 of them
+    const float *Ainv;
+};
+template <int NL>
+__global__ __launch_bounds__(16 * CG_TAIL) void k_cg_tail(CgTail T) {
+    __shared__ float M[2 * CG_DENSE * (2 * CG_DENSE + 1)];
+    __shared__ float2 x0[NL > 0 ? 16 * CG_TAIL : 1], x1[NL > 1 ? CG_TAIL : 1], rd[CG_DENSE], ed[CG_DENSE];
+    const int t = threadIdx.x, P = t >> 4, sub = t & 15;
+    const CoarseLevel &C = T.lev[NL];
+    const int n = 2 * C.ax * C.ay;
+    float4 B[NL > 0 ? NL : 1][9];
+    float2 r[NL > 0 ? NL : 1], e[NL > 0 ? NL : 1], dl[NL > 0 ? NL : 1];
+    int ci[NL > 0 ? NL : 1], cj[NL > 0 ? NL : 1], c[NL > 0 ? NL : 1];   // this lane's child (c < 0: none)
 #pragma unroll
-    for (int d = 0; d < 9; ++d) {
-        const int nb = cg_nb(ci, cj, ax, ay, d % 3 - 1, d / 3 - 1, periodic);
-        if (nb < 0) continue;
-        const float4 B = Ab[d];
-        const float2 en = corr(nb);
-        ru -= B.x * en.x + B.y * en.y;
-        rv -= B.z * en.x + B.w * en.y;
+    for (int l = 0; l < NL; ++l) {
+        const CoarseLevel &F = T.lev[l];
+        const int axp = T.lev[l + 1].ax;
+        ci[l] = CG_AGG * (P % axp) + (sub & 3);
+        cj[l] = CG_AGG * (P / axp) + (sub >> 2);
+        c[l] = ci[l] < F.ax && cj[l] < F.ay ? ci[l] + F.ax * cj[l] : -1;   // cj >= ay past the last parent
+        r[l] = e[l] = dl[l] = make_float2(0.0f, 0.0f);
+        if (c[l] < 0) continue;
+#pragma unroll
+        for (int d = 0; d < 9; ++d) B[l][d] = reinterpret_cast<const float4 *>(F.A + c[l] * 36)[d];
+        dl[l] = reinterpret_cast<const float2 *>(F.dl1)[c[l]];
     }
-    reinterpret_cast<float2 *>(eo)[c] = make_float2(ec.x + dl1[2 * c] * ru, ec.y + dl1[2 * c + 1] * rv);
+    if constexpr (NL > 0) {
+        if (c[0] >= 0) {
+            r[0] = reinterpret_cast<const float2 *>(T.lev[0].r)[c[0]];
+            e[0] = reinterpret_cast<const float2 *>(T.lev[0].e)[c[0]];
+            x0[c[0]] = e[0];
+        }
+    } else {
+        if (t < C.ax * C.ay) rd[t] = reinterpret_cast<const float2 *>(C.r)[t];
+    }
+    for (int w = t; w < n * n; w += blockDim.x) M[w / n * (n + 1) + w % n] = T.Ainv[w];   // n is even
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+        const CoarseLevel &F = T.lev[l], &G = T.lev[l + 1];
+        const float2 *x = l ? x1 : x0;
+        float2 s = make_float2(0.0f, 0.0f);
+        if (c[l] >= 0) {
+            s = r[l];
+            cg_sub_row(ci[l], cj[l], F.ax, F.ay, T.periodic, B[l], [&](int nb) { return x[nb]; }, s);
+        }
+        s = make_float2(cg_sum16(s.x), cg_sum16(s.y));
+        if (sub == 0 && P < G.ax * G.ay) {
+            if (l + 1 < NL) x1[P] = s;
+            else rd[P] = s;
+        }
+        __syncthreads();
+        if (l + 1 < NL) {   // the next level's residual to its lanes, its pre-smoothed e in its place
+            if (c[NL - 1] >= 0) {
+                r[NL - 1] = x1[c[NL - 1]];
+                e[NL - 1] = make_float2(dl[NL - 1].x * r[NL - 1].x, dl[NL - 1].y * r[NL - 1].y);
+                x1[c[NL - 1]] = e[NL - 1];   // each entry has one lane
+            }
+            __syncthreads();
+        }
+    }
+    if (t < n) {
+        const float *rv = reinterpret_cast<const float *>(rd);
+        float s = 0.0f;
+        for (int j = 0; j < n; ++j) s += M[t * (n + 1) + j] * rv[j];
+        if (NL > 0) reinterpret_cast<float *>(ed)[t] = s;
+        else C.eo[t] = s;
+    }
+#pragma unroll
+    for (int l = NL - 1; l >= 0; --l) {
+        const CoarseLevel &F = T.lev[l], &G = T.lev[l + 1];
+        float2 *x = l ? x1 : x0;
+        const float2 *xp = l + 1 < NL ? x1 : ed;
+        __syncthreads();
+        if (c[l] >= 0) {
+            const float2 y = xp[ci[l] / CG_AGG + G.ax * (cj[l] / CG_AGG)];
+            e[l] = make_float2(e[l].x + y.x, e[l].y + y.y);
+            x[c[l]] = e[l];
+        }
+        __syncthreads();
+        if (c[l] >= 0) cg_sub_row(ci[l], cj[l], F.ax, F.ay, T.periodic, B[l], [&](int nb) { return x[nb]; }, r[l]);
+        const float2 o = make_float2(e[l].x + dl[l].x * r[l].x, e[l].y + dl[l].y * r[l].y);
+        if (l) {
+            __syncthreads();   // every lane has read its neighbours
+            if (c[l] >= 0) x[c[l]] = o;
+        } else if (c[l] >= 0) {
+            reinterpret_cast<float2 *>(F.eo)[c[l]] = o;
+        }
+    }
+}
+
+// the first level of the V-cycle's coarse end
+static int cg_tail_first(const CoarseHier *h) {
+    int l = h->nlev - 1;
+    while (l > 0 && (long long)h->lev[l].ax * h->lev[l].ay <= CG_TAIL) --l;
+    return l;
 }
 
 // z += P e1 on every node of an owned active column and of its periodic halo images
@@ -573,7 +671,9 @@ static int coarse_alloc(cism_ctx *c) {
         const size_t n = (size_t)L.ax * L.ay;
         e = hipMalloc(&L.A64, sizeof(double) * 36 * n);
         if (e == hipSuccess) e = hipMalloc(&L.A, sizeof(float) * 36 * n);
-        float **vs[] = {&L.dl1, &L.r, &L.e, &L.eo};
+        if (e == hipSuccess) e = hipMalloc(&L.dl1, sizeof(float) * 2 * n);
+        if (l > cg_tail_first(h)) continue;   // vectors in LDS
+        float **vs[] = {&L.r, &L.e, &L.eo};
         for (float **p : vs)
             if (e == hipSuccess) e = hipMalloc(p, sizeof(float) * 2 * n);
     }
@@ -665,15 +765,19 @@ int coarse_apply(cism_ctx *c, float *z) {
     const long long n1 = (long long)lv[0].ax * lv[0].ay;
     hipLaunchKernelGGL(k_cg_restrict1, dim3(nblocks_for(16 * n1)), dim3(CISM_BLOCK), 0, c->stream, g, c->av, h->colsum,
                        lv[0].ax, lv[0].ay, L > 1, lv[0].dl1, lv[0].r, lv[0].e);
-    for (int l = 0; l + 1 < L; ++l) {
+    const int tl = cg_tail_first(h), nt = L - 1 - tl;
+    for (int l = 0; l < tl; ++l) {
         const long long np = (long long)lv[l + 1].ax * lv[l + 1].ay;
         hipLaunchKernelGGL(k_cg_down, dim3(nblocks_for(16 * np)), dim3(CISM_BLOCK), 0, c->stream, lv[l].ax, lv[l].ay,
                            lv[l + 1].ax, lv[l + 1].ay, g.periodic, lv[l].A, lv[l].r, lv[l].e, l + 2 < L,
                            lv[l + 1].dl1, lv[l + 1].r, lv[l + 1].e);
     }
-    const CoarseLevel &C = lv[L - 1];
-    hipLaunchKernelGGL(k_cg_dense_apply, dim3(1), dim3(64), 0, c->stream, 2 * C.ax * C.ay, h->Ainv, C.r, C.eo);
-    for (int l = L - 2; l >= 0; --l) {
+    CgTail tail{g.periodic, {}, h->Ainv};
+    for (int l = tl; l < L; ++l) tail.lev[l - tl] = lv[l];
+    const unsigned threads = nt ? std::max(256, (16 * lv[tl + 1].ax * lv[tl + 1].ay + 63) / 64 * 64) : 256;
+    hipLaunchKernelGGL(nt == 0 ? k_cg_tail<0> : nt == 1 ? k_cg_tail<1> : k_cg_tail<2>, dim3(1), dim3(threads), 0,
+                       c->stream, tail);
+    for (int l = tl - 1; l >= 0; --l) {
         const long long n = (long long)lv[l].ax * lv[l].ay;
         hipLaunchKernelGGL(k_cg_up, dim3(nblocks_for(n)), dim3(CISM_BLOCK), 0, c->stream, lv[l].ax, lv[l].ay,
                            lv[l + 1].ax, g.periodic, lv[l].A, lv[l].r, lv[l].e, lv[l + 1].eo, lv[l].dl1, lv[l].eo);
