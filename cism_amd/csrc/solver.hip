@@ -921,7 +921,7 @@ int launch_halo_mat(cism_ctx *c, double *A) {
 // second launch updates x and r, and with the diagonal or no preconditioner forms the next
 // z and the partials of (r, z) too.  Both form their scalar from the partials they need
 // (red_sums).  35 x 35 x 10, diagonal preconditioner: an iteration was 10 launches of 2.4 to
-// 6 us, 42 us in all (187 ms a solve); two take 12.2 + 4.1 us, 24 us with the checks (105 ms).
+// 6 us, 42 us in all (187 ms a solve); two take 7.9 + 4.1 us (88 ms a solve, checks included).
 
 // beta = (r, z) / the last (r, z)   (pcg:366-382)
 __device__ inline CgState std_beta_step(CgState st, double s0) {
@@ -938,6 +938,22 @@ __device__ inline CgState std_alpha_step(CgState st, double s0) {
     return st;
 }
 
+// The new direction of a block's nodes and their neighbours is formed once, in LDS: a window
+// of W = CISM_BLOCK + 2 nodes (a level more at each end) per row of columns, widened by a
+// column each way, or, when a column is longer than W, nine windows of W, one per column
+// direction, which are then the shorter of the two.  The windows' z and d are on their way
+// while the scalar is formed.  Bound: at small sizes the latency of the scalar and of three
+// groups of matrix loads in one wave per SIMD, at large ones the matrix from past L2.  Formed
+// 27 times a node instead: 12.0 us at 35 x 35 x 10 (7.9 here); an iteration at 31 x 31 x 10
+// 14.2 us (10.0), 120 x 130 x 11 61 us (53), 400 x 410 x 11 453 us (391), 400 x 410 x 2 103 us
+// (89), 40 x 40 x 60 40 us (33).
+#define STD_AHEAD 4   // entries per lane loaded ahead: all of three windows to 41 levels
+__host__ __device__ inline bool std_three_windows(int nz) { return nz <= CISM_BLOCK + 2; }
+inline size_t std_window_entries(int nz) {
+    const size_t W = CISM_BLOCK + 2;
+    return std_three_windows(nz) ? 3 * (W + 2 * nz) : 9 * W;   // at most 37 KB of FP64 pairs
+}
+
 template <typename T, typename M>
 __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned chunk, const M A,
                                                            const int32_t *__restrict__ av,
@@ -948,6 +964,32 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned c
     using V2 = typename Vec2<T>::t;
     const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;
     if (M::xcd && lb * blockDim.x >= g.nn) return;
+    const int nz = g.nz, W = CISM_BLOCK + 2;
+    const bool nine = !std_three_windows(nz);
+    const int L = nine ? W : W + 2 * nz, total = (nine ? 9 : 3) * L;
+    const long long q0 = lb * CISM_BLOCK;
+    extern __shared__ __align__(16) char staged[];
+    V2 *D = reinterpret_cast<V2 *>(staged);
+    // the node whose z and d make entry e: the image of entry e's own, or -1
+    auto source = [&](int e) -> long long {
+        const int w = nine ? e / L : (e >= L) + (e >= 2 * L);
+        const long long off = nine ? nz * ((w % 3 - 1) + (long long)g.sx * (w / 3 - 1))
+                                   : nz * ((long long)g.sx * (w - 1) - 1);
+        const long long n = q0 - 1 + off + (e - w * L);
+        if (e >= total || n < 0 || n >= g.nn) return -1;
+        const int col = node_col(g, n);
+        const int im = halo_image(col_i(g, col), g.sx, g.periodic), jm = halo_image(col_j(g, col), g.sy, g.periodic);
+        return im >= 0 && jm >= 0 ? nz * (im + (long long)g.sx * jm) + (n - (long long)nz * col) : -1;
+    };
+    V2 zz[STD_AHEAD], dd[STD_AHEAD];
+    bool has[STD_AHEAD];
+#pragma unroll
+    for (int u = 0; u < STD_AHEAD; ++u) {
+        const long long p = source(threadIdx.x + u * CISM_BLOCK);
+        has[u] = p >= 0;
+        zz[u] = reinterpret_cast<const V2 *>(z)[has[u] ? p : 0];
+        dd[u] = reinterpret_cast<const V2 *>(d)[has[u] ? p : 0];
+    }
     __shared__ double sb;
     {
         double s[1];
@@ -960,32 +1002,36 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned c
         __syncthreads();
     }
     const T beta = (T)sb;
+    auto dir = [&](bool in, const V2 &zv, const V2 &dv) {
+        V2 v;
+        v.x = in ? zv.x + beta * dv.x : (T)0;
+        v.y = in ? zv.y + beta * dv.y : (T)0;
+        return v;
+    };
+#pragma unroll
+    for (int u = 0; u < STD_AHEAD; ++u) {
+        const int e = threadIdx.x + u * CISM_BLOCK;
+        if (e < total) D[e] = dir(has[u], zz[u], dd[u]);
+    }
+    for (int e = threadIdx.x + STD_AHEAD * CISM_BLOCK; e < total; e += CISM_BLOCK) {
+        const long long p = source(e);
+        D[e] = dir(p >= 0, reinterpret_cast<const V2 *>(z)[p >= 0 ? p : 0],
+                   reinterpret_cast<const V2 *>(d)[p >= 0 ? p : 0]);
+    }
+    __syncthreads();
     double acc[1] = {0.0};
-    const long long q = lb * blockDim.x + threadIdx.x;
+    const long long q = q0 + threadIdx.x;
     if (q < g.nn) {
         const int k = node_level(g, q);
         const long long col = node_col(g, q);
         const int i = col_i(g, col), j = col_j(g, col);
-        // the first node of the image of a column, or -1
-        auto image = [&](int ii, int jj) {
-            const int im = halo_image(ii, g.sx, g.periodic), jm = halo_image(jj, g.sy, g.periodic);
-            return im >= 0 && jm >= 0 ? (long long)g.nz * (im + (long long)g.sx * jm) : -1;
+        // entry of the neighbour in column direction o of this lane's node
+        auto entry = [&](int o) {
+            return threadIdx.x + 1 + (nine ? o * W : (o / 3) * L + (o % 3) * nz);
         };
-        // the new d of level kk of an image column (0 without one); every load unconditional
-        auto dir = [&](long long base, int kk) {
-            const long long p = (base >= 0 ? base : 0) + kk;
-            const V2 zz = reinterpret_cast<const V2 *>(z)[p], dd = reinterpret_cast<const V2 *>(d)[p];
-            V2 v;
-            v.x = base >= 0 ? zz.x + beta * dd.x : (T)0;
-            v.y = base >= 0 ? zz.y + beta * dd.y : (T)0;
-            return v;
-        };
-        const V2 own = dir(image(i, j), k);
+        const V2 own = D[entry(4)];
         T su = 0, sv = 0;
         if (is_owned(g, i, j) && av[col]) {
-            long long nb[9];
-#pragma unroll
-            for (int o = 0; o < 9; ++o) nb[o] = image(i + o % 3 - 1, j + o / 3 - 1);
             // the row product's order and operations (row_product)
 #pragma unroll
             for (int kA = -1; kA <= 1; ++kA) {
@@ -993,7 +1039,7 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned c
 #pragma unroll
                 for (int o = 0; o < 9; ++o) {
                     const int iA = o % 3 - 1, jA = o / 3 - 1;
-                    const V2 xx = dir(nb[o], k + kA);
+                    const V2 xx = D[entry(o) + kA];
                     T uu, uv, vu, vv;
                     A.blocks(q, slot_of(iA, jA, kA), q + kA + (long long)g.nz * (iA + (long long)g.sx * jA), uu, uv,
                              vu, vv);
@@ -1462,7 +1508,8 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
                                    d, v.q, v.x, v.r, v.z, RedSrc{}, c->sc, cur, c->partials);
             }
             const RedSrc s1 = red_source<1>(c, c->partials, nb);
-            hipLaunchKernelGGL((k_std_matvec<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
+            hipLaunchKernelGGL((k_std_matvec<T, M>), dim3(nbv), dim3(CISM_BLOCK),
+                               std_window_entries(g.nz) * sizeof(typename Vec2<T>::t), c->stream, g, chunk, A, c->av,
                                v.z, d, dn, v.q, s1, c->sc, cur, mpart);
             cur ^= 1;
             std::swap(d, dn);
