@@ -361,7 +361,7 @@ def main(argv=None):
                      "frac_fp64_peak": round(asm_tflops / FP64_VALU_PEAK_TFLOPS, 4)},
         "roofline": {"bound": "hbm", "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs32 / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_matvec_dots<float,2,MatSym32>",
+                     "kernel": "k_matvec_dots<float, MatSym32>",
                      "algorithmic_bytes_per_launch": bytes32},
         "cpu_baseline": cpu,
         "cpu_baseline_all_cores": cpu_all,
