@@ -961,6 +961,9 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_std_matvec(GridDev g, unsigned c
                                                            T *__restrict__ dn, T *__restrict__ y, RedSrc src,
                                                            DevScal *__restrict__ sc, int cur,
                                                            double *__restrict__ partials) {
+    // its partials are in node-block order, which mpart32 does not hold: the places past a
+    // grid's last block would no longer be zero for the sums over xcd_slots_for(nn) of them
+    static_assert(!M::slots, "partials in node-block order");
     using V2 = typename Vec2<T>::t;
     const long long lb = M::xcd ? xcd_block(chunk) : (long long)blockIdx.x;
     if (M::xcd && lb * blockDim.x >= g.nn) return;
@@ -1439,6 +1442,10 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
         cism_set_error("the coarse correction is a preconditioner of the FP32 inner solves only");
         return CISM_ERR_ARG;
     }
+    if (M::slots && !chrongear) {
+        cism_set_error("the FP32 inner solves are Chron-Gear only");
+        return CISM_ERR_ARG;
+    }
     if (precond >= 2) {
         TimerRange r_p("pcg_precond_init", c->stream, true);
         if constexpr (std::is_same<M, MatSym32>::value && std::is_same<T, float>::value) {
@@ -1491,37 +1498,39 @@ static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precon
     };
     bool done = false;
     if (!chrongear) {
-        // pcg:253-304: halo x, r = b - A x (no halo on r)
-        CISM_TRY((launch_halo_t<T, false>(c, v.x)));
-        hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
-                           v.x, v.b, v.r, 0, c->partials);
-        T *d = v.d, *dn = v.Az;   // the direction and where the next one goes
-        for (int n = 1; n <= maxiters && !done; ++n) {
-            // z and (r, z): with a point preconditioner the last update has formed them
-            // unless the check has replaced r since
-            if (precond >= 2) {
-                CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
-                hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, v.r, v.z,
-                                   c->partials);
-            } else if (n % 5 == 1) {
-                hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 0,
-                                   d, v.q, v.x, v.r, v.z, RedSrc{}, c->sc, cur, c->partials);
-            }
-            const RedSrc s1 = red_source<1>(c, c->partials, nb);
-            hipLaunchKernelGGL((k_std_matvec<T, M>), dim3(nbv), dim3(CISM_BLOCK),
-                               std_window_entries(g.nz) * sizeof(typename Vec2<T>::t), c->stream, g, chunk, A, c->av,
-                               v.z, d, dn, v.q, s1, c->sc, cur, mpart);
-            cur ^= 1;
-            std::swap(d, dn);
-            const RedSrc s2 = red_source<1>(c, mpart, nbr);
-            hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 1, d,
-                               v.q, v.x, v.r, v.z, s2, c->sc, cur, c->partials);
-            cur ^= 1;
-            HIP_TRY(hipGetLastError());
-            checked = false;
-            if (n % 5 == 0) {
-                if (check == 0) CISM_TRY((launch_halo_t<T, false>(c, v.x)));
-                CISM_TRY(check_conv(n, done));
+        if constexpr (!M::slots) {
+            // pcg:253-304: halo x, r = b - A x (no halo on r)
+            CISM_TRY((launch_halo_t<T, false>(c, v.x)));
+            hipLaunchKernelGGL((k_residual<T, M>), dim3(nbv), dim3(CISM_BLOCK), 0, c->stream, g, chunk, A, c->av,
+                               v.x, v.b, v.r, 0, c->partials);
+            T *d = v.d, *dn = v.Az;   // the direction and where the next one goes
+            for (int n = 1; n <= maxiters && !done; ++n) {
+                // z and (r, z): with a point preconditioner the last update has formed them
+                // unless the check has replaced r since
+                if (precond >= 2) {
+                    CISM_TRY((launch_precond<T, M>(c, precond, A, v.F, v.r, v.z)));
+                    hipLaunchKernelGGL(k_dot<T>, dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, v.r, v.z,
+                                       c->partials);
+                } else if (n % 5 == 1) {
+                    hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 0,
+                                       d, v.q, v.x, v.r, v.z, RedSrc{}, c->sc, cur, c->partials);
+                }
+                const RedSrc s1 = red_source<1>(c, c->partials, nb);
+                hipLaunchKernelGGL((k_std_matvec<T, M>), dim3(nbv), dim3(CISM_BLOCK),
+                                   std_window_entries(g.nz) * sizeof(typename Vec2<T>::t), c->stream, g, chunk, A, c->av,
+                                   v.z, d, dn, v.q, s1, c->sc, cur, mpart);
+                cur ^= 1;
+                std::swap(d, dn);
+                const RedSrc s2 = red_source<1>(c, mpart, nbr);
+                hipLaunchKernelGGL((k_std_update<T, M>), dim3(nb), dim3(CISM_BLOCK), 0, c->stream, g, A, precond, 1, d,
+                                   v.q, v.x, v.r, v.z, s2, c->sc, cur, c->partials);
+                cur ^= 1;
+                HIP_TRY(hipGetLastError());
+                checked = false;
+                if (n % 5 == 0) {
+                    if (check == 0) CISM_TRY((launch_halo_t<T, false>(c, v.x)));
+                    CISM_TRY(check_conv(n, done));
+                }
             }
         }
     } else {

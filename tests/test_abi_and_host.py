@@ -50,6 +50,19 @@ def test_noalloc_entry_point_rejects_bad_sizes_before_any_gpu_call():
     assert f(40, 40, 11, 1, 0, None, *([None] * 12)) == 5   # null arrays
 
 
+def test_no_standard_pcg_on_the_fp32_matrix():
+    """The FP32 matvec's dot partials lie in a buffer whose places past the grid's last block
+    stay zero; the standard PCG's matvec stores its partials in another order and would fill
+    them, so that every later inner solve of the context summed wrong.  The inner solves are
+    Chron-Gear: the library holds no standard-PCG kernel for the FP32 matrix."""
+    path = os.path.join(ROOT, "cism_amd", "libcism_gpu.so")
+    if not os.path.exists(path):
+        pytest.fail("libcism_gpu.so is not built (run __graft_entry__.build())")
+    kernels = [n for n in os.popen(f"nm -DC {path}").read().splitlines() if "k_std_" in n]
+    assert any("MatSym64" in n for n in kernels) and any("MatFull" in n for n in kernels)
+    assert not [n for n in kernels if "MatSym32" in n]
+
+
 def test_fortran_shim_exports():
     path = os.path.join(ROOT, "cism_amd", "libcism_fortran.so")
     if not os.path.exists(path):
