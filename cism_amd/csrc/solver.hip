@@ -647,10 +647,10 @@ __global__ __launch_bounds__(128) void k_sia_setup_sym32(GridDev g, const float 
 }
 
 // One column and component of the SIA preconditioner: the Thomas substitutions
-// on s (level k at s[2k]) with the factors precomputed by k_sia_setup.  For
-// nz <= 24 the factors are first loaded into registers (sia_factors), so that a
-// caller can issue those loads early; the substitutions would otherwise wait on
-// one global load per level.
+// on s (level k at s[2k]) with the factors precomputed by k_sia_setup: from registers
+// (sia_factors, sia_solve), so that a caller can issue those loads early where the
+// substitutions would otherwise wait on one global load per level, or from memory
+// (sia_column_mem), which leaves the registers to more waves.
 template <typename T, int NZMAX>
 struct SiaFactors {
     T fs[NZMAX], fb[NZMAX], fg[NZMAX];
@@ -689,6 +689,24 @@ __device__ __forceinline__ void sia_solve(int nz, const SiaFactors<T, NZMAX> &f,
         }
 }
 
+template <typename T>
+__device__ __forceinline__ void sia_column_mem(int nz, long long ncol, const T *__restrict__ F, long long col,
+                                               int comp, T *s) {
+    const T *sb = F + (long long)(0 * 2 + comp) * nz * ncol + col;
+    const T *be = F + (long long)(1 * 2 + comp) * nz * ncol + col;
+    const T *ga = F + (long long)(2 * 2 + comp) * nz * ncol + col;
+    T prev = s[0] / be[0];
+    s[0] = prev;
+    for (int k = 1; k < nz; ++k) {
+        prev = (s[2 * k] - sb[k * ncol] * prev) / be[k * ncol];
+        s[2 * k] = prev;
+    }
+    for (int k = nz - 2; k >= 0; --k) {
+        prev = s[2 * k] - ga[(k + 1) * ncol] * prev;
+        s[2 * k] = prev;
+    }
+}
+
 template <typename T, int NZMAX>
 __device__ __forceinline__ void sia_column(int nz, long long ncol, const T *__restrict__ F, long long col,
                                            int comp, T *s) {
@@ -697,19 +715,7 @@ __device__ __forceinline__ void sia_column(int nz, long long ncol, const T *__re
         sia_factors<T, NZMAX>(nz, ncol, F, col, comp, f);
         sia_solve<T, NZMAX>(nz, f, s);
     } else {
-        const T *sb = F + (long long)(0 * 2 + comp) * nz * ncol + col;
-        const T *be = F + (long long)(1 * 2 + comp) * nz * ncol + col;
-        const T *ga = F + (long long)(2 * 2 + comp) * nz * ncol + col;
-        T prev = s[0] / be[0];
-        s[0] = prev;
-        for (int k = 1; k < nz; ++k) {
-            prev = (s[2 * k] - sb[k * ncol] * prev) / be[k * ncol];
-            s[2 * k] = prev;
-        }
-        for (int k = nz - 2; k >= 0; --k) {
-            prev = s[2 * k] - ga[(k + 1) * ncol] * prev;
-            s[2 * k] = prev;
-        }
+        sia_column_mem<T>(nz, ncol, F, col, comp, s);
     }
 }
 
@@ -1223,6 +1229,12 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update(GridDev g, const T *__
 // FUSED: the workgroup forms the scalars itself, with its first node's vectors under way.  Without
 // it (many workgroups, k_cg_scalars before) the kernel keeps to 68 registers at FP32 and 12
 // levels instead of 97: 551 ms a 1200 x 1400 x 11 solve, 563 with them.
+//
+// The column factors are in registers, loaded first, to 12 levels, and to 24 where FUSED; past
+// that they come from memory.  Linear part of two Picard iterations of 100 steps, FP64,
+// registers against memory: FUSED 96 x 96 x 13 6.72 / 7.01 ms, 160 x 160 x 21 22.5 / 23.0,
+// 256 x 256 x 21 57.7 / 54.8; not FUSED 400 x 400 x 16 101.8 / 98.9, 500 x 500 x 16 157.1 / 152.8,
+// 600 x 640 x 21 317.6 / 312.4; a mixed solve at 400 x 400 x 16 85.8 / 81.7.
 template <typename T, int NZMAX, bool FUSED>
 __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T *__restrict__ Az,
                                                        T *__restrict__ d, T *__restrict__ qv,
@@ -1244,8 +1256,9 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
     const int comp = (threadIdx.x >> 6) & 1, lc = threadIdx.x & 63;
     const long long col = col0 + lc;
     const bool solve = threadIdx.x < 128 && lc < ncols && av[col];
-    SiaFactors<T, (NZMAX <= 24 ? NZMAX : 1)> f;
-    if constexpr (NZMAX <= 24)
+    constexpr bool REGS = NZMAX <= (FUSED ? 24 : 12);
+    SiaFactors<T, (REGS ? NZMAX : 1)> f;
+    if constexpr (REGS)
         if (solve) sia_factors<T, NZMAX>(nz, ncol, F, col, comp, f);
     // node t of the block: level t % nz of local column t / nz (32-bit: the context
     // limits grids to 2^30 nodes).
@@ -1287,8 +1300,8 @@ __global__ __launch_bounds__(256) void k_cg_update_sia(GridDev g, T *z, const T 
                 colsum[2 * col + comp] = cs;
             }
         }
-        if constexpr (NZMAX <= 24) sia_solve<T, NZMAX>(nz, f, sr + 2 * lc * nz + comp);
-        else sia_column<T, NZMAX>(nz, ncol, F, col, comp, sr + 2 * lc * nz + comp);
+        if constexpr (REGS) sia_solve<T, NZMAX>(nz, f, sr + 2 * lc * nz + comp);
+        else sia_column_mem<T>(nz, ncol, F, col, comp, sr + 2 * lc * nz + comp);
     }
     __syncthreads();
     for (int t = threadIdx.x; t < 2 * nn; t += blockDim.x)
