@@ -46,10 +46,25 @@ static int scratch_on_device(int device, double **out) {
     return CISM_OK;
 }
 
+// division of an n < 2^31 by a divisor fixed for a launch, exact: n m >> s with
+// m = ceil(2^s / d), s = 31 + ceil(log2 d)
+struct FastDiv {
+    unsigned m;
+    int s;
+    explicit FastDiv(unsigned d) {
+        int l = 0;
+        while ((1ULL << l) < d) ++l;
+        s = 31 + l;
+        m = (unsigned)(((1ULL << s) + d - 1) / d);
+    }
+    __device__ int operator()(int n) const { return (int)(((unsigned long long)(unsigned)n * m) >> s); }
+};
+
 struct FGrid {
     int nz, sx, sy;            // levels, staggered extents (nx-1, ny-1)
     int ilo, ihi, jlo, jhi;    // owned staggered vertices, 0-based inclusive
-    long long nn;
+    int nn;                    // nodes, at most 2^30
+    FastDiv by_nz, by_sx;
 };
 
 // r = A x - b on owned active rows, 0 elsewhere; the 27 slots summed in indxA order as the
@@ -57,16 +72,24 @@ struct FGrid {
 // for bit.  part[2 * block + {0, 1}] = the block's |r|^2 and |b|^2 over owned active rows, in a
 // fixed order.
 //
-// Bound: one read of the four blocks, 864 of the 912 bytes a node needs.  In the Fortran layout
-// a node's 27 coefficients of a block are 216 contiguous bytes, so lanes that walk their own
-// rows touch 64 lines per load and fetch every line again for most of the 27 slots (2.9 ms,
-// 0.78 TB/s, at 503 x 453 x 11).  Here a workgroup is one wave and takes tiles of 64 nodes: it
-// loads the tile's two blocks of one row (Auu, Auv, then Avu, Avv) as contiguous runs into
-// registers, passes them through LDS (27.6 KB, four or five waves per CU; the stride of 27
-// doubles is odd, so the row reads are conflict-free) and loads the next pair while it sums
-// this one: 110 KB per CU in flight.  0.50 ms at that size with three quarters of the columns
-// active (21.7 -> 13.5 us a call at 34 x 34 x 10).  A tile without an owned active node is
-// not read.
+// Bound: one read of the four blocks, 864 of the 912 bytes a node needs, and on small grids
+// the fetch of the code, which each wave runs once.  In the Fortran layout a node's 27
+// coefficients of a block are 216 contiguous bytes, so lanes that walk their own rows touch 64
+// lines per load and fetch every line again for most of the 27 slots.  Here a workgroup is one
+// wave and takes tiles of 64 nodes, each in two steps, one per component: a step's two blocks
+// (Auu, Auv, then Avu, Avv) are loaded as contiguous runs into registers while the step before
+// sums, and pass through LDS (27.6 KB, five waves per CU; the stride of 27 doubles is odd, so the
+// row reads are conflict-free).  The solution at a node's neighbours is loaded once for both
+// components.  The two steps are one rolled loop, the divisions multiplications and, with one
+// level, the 18 slots without a neighbour are not run through: 7 KB of code instead of 15.
+// A tile without an owned active node is not read.
+//
+// A lane per node on its own row / tiles with both components written out and the solution
+// loaded for each / now, us a call, three quarters of the columns active (all of them at one
+// level): 19 x 19 x 1 nodes 8.6 / 10.0 / 8.7, 11 x 11 x 2 10.3 / 12.1 / 9.5, 34 x 34 x 10 17.4 / 12.4 / 9.6,
+// 103 x 103 x 11 93 / 32 / 23, 503 x 453 x 11 2915 / 512 / 364; 34 x 34 x 10 with 5 % of the columns active
+// 11.1 / 12.3 / 10.1.  Only a large grid without any row is slower than with a lane per node,
+// whose waves are more: 503 x 453 x 11 15.6 / 26.3 / 22.8.
 // W doubles per load: 2 when the four blocks are 16-byte aligned (a tile starts at a
 // multiple of 13,824 bytes), else 1.
 template <int W>
@@ -75,55 +98,39 @@ struct RowPair {
     double a[N][W], b[N][W];
 };
 
+// count coefficients of blocks A and B; past them a lane reads the last ones again.  The last
+// of an odd count with W = 2 is left to pair_stage.
 template <int W>
 __device__ __forceinline__ void pair_load(RowPair<W> &R, const double *__restrict__ A, const double *__restrict__ B,
-                                          long long q0, int count, int lane) {
+                                          int count, int lane) {
     typedef double vec __attribute__((ext_vector_type(W)));
-    const double *pa = A + 27 * q0, *pb = B + 27 * q0;
+    const int last = (count - W) / W * W;
 #pragma unroll
     for (int t = 0; t < RowPair<W>::N; ++t) {
-        const int e = (t * 64 + lane) * W;
-        if (e + W <= count) {
-            const vec va = *reinterpret_cast<const vec *>(pa + e), vb = *reinterpret_cast<const vec *>(pb + e);
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                R.a[t][w] = va[w];
-                R.b[t][w] = vb[w];
-            }
-        } else if (e < count) {   // the odd last value of the grid
-            R.a[t][0] = pa[e];
-            R.b[t][0] = pb[e];
-        }
-    }
-}
-
-template <>
-__device__ __forceinline__ void pair_load<1>(RowPair<1> &R, const double *__restrict__ A,
-                                             const double *__restrict__ B, long long q0, int count, int lane) {
-    const double *pa = A + 27 * q0, *pb = B + 27 * q0;
-#pragma unroll
-    for (int t = 0; t < RowPair<1>::N; ++t) {
-        const int e = t * 64 + lane;
-        if (e < count) {
-            R.a[t][0] = pa[e];
-            R.b[t][0] = pb[e];
-        }
+        const int e = min((t * 64 + lane) * W, last);
+        *reinterpret_cast<vec *>(R.a[t]) = *reinterpret_cast<const vec *>(A + e);
+        *reinterpret_cast<vec *>(R.b[t]) = *reinterpret_cast<const vec *>(B + e);
     }
 }
 
 // the pair to LDS, slot-minor as in memory; a lane's row is then S[27 * lane ..]
 template <int W>
-__device__ __forceinline__ void pair_stage(const RowPair<W> &R, double *__restrict__ SA, double *__restrict__ SB,
-                                           int lane) {
+__device__ __forceinline__ void pair_stage(const RowPair<W> &R, const double *__restrict__ A,
+                                           const double *__restrict__ B, int count, double *__restrict__ SA,
+                                           double *__restrict__ SB, int lane) {
 #pragma unroll
     for (int t = 0; t < RowPair<W>::N; ++t) {
         const int e = (t * 64 + lane) * W;
-        if (e < 27 * 64)
+        if (e + W <= count)
 #pragma unroll
             for (int w = 0; w < W; ++w) {
                 SA[e + w] = R.a[t][w];
                 SB[e + w] = R.b[t][w];
             }
+    }
+    if (W == 2 && (count & 1) && lane == 0) {
+        SA[count - 1] = A[count - 1];
+        SB[count - 1] = B[count - 1];
     }
 }
 
@@ -135,31 +142,25 @@ __global__ __launch_bounds__(64) void k_resvec_fortran(
     double *__restrict__ ru, double *__restrict__ rv, double *__restrict__ part) {
     __shared__ alignas(16) double SA[27 * 64], SB[27 * 64];
     const int lane = threadIdx.x;
-    const long long cst = g.nz, rst = (long long)g.nz * g.sx;
-    const int ntiles = (int)((g.nn + 63) / 64);
+    const int cst = g.nz, rst = g.nz * g.sx;
+    const int ntiles = (g.nn + 63) / 64;
     double acc[2] = {0.0, 0.0};
-    RowPair<W> R = {};
-    // this lane's node of a tile: whether it has a row, and its level
+    // whether this lane's node of a tile has a row, and its level
     auto row_of = [&](int tile, int &k) {
-        const long long q = (long long)tile * 64 + lane;
-        if (q >= g.nn) return false;
-        const int qi = (int)q, col = qi / g.nz;   // grids end at 2^30 nodes
-        k = qi - col * g.nz;
-        const int j = col / g.sx, i = col - j * g.sx;
-        return i >= g.ilo && i <= g.ihi && j >= g.jlo && j <= g.jhi && av[col] != 0;
+        const int q = tile * 64 + lane;
+        const bool in = tile < ntiles && q < g.nn;
+        const int col = in ? g.by_nz(q) : 0, j = g.by_sx(col), i = col - j * g.sx;
+        k = q - col * g.nz;
+        return av[col] != 0 && in && i >= g.ilo && i <= g.ihi && j >= g.jlo && j <= g.jhi;
     };
-    auto count_of = [&](int tile) {
-        const long long left = g.nn - (long long)tile * 64;
-        return (int)(left < 64 ? left : 64) * 27;
-    };
-    // the next tile with a row from `tile` on; the rowless ones before it are written here
-    bool row = false;
-    int k = 0;
-    auto find = [&](int tile) {
-        for (; tile < ntiles; tile += gridDim.x) {
+    // the next tile with a row from `tile` on; the rowless ones before it are written here, each
+    // after the vertices of the tile behind it are on their way
+    auto find = [&](int tile, bool &row, int &k) {
+        row = row_of(tile, k);
+        while (tile < ntiles && !__any(row)) {
+            const int q = tile * 64 + lane;
+            tile += gridDim.x;
             row = row_of(tile, k);
-            if (__any(row)) break;
-            const long long q = (long long)tile * 64 + lane;
             if (q < g.nn) {
                 ru[q] = 0.0;
                 rv[q] = 0.0;
@@ -167,50 +168,73 @@ __global__ __launch_bounds__(64) void k_resvec_fortran(
         }
         return tile;
     };
-    // one component's row product from the staged pair, slots in indxA order
-    auto product = [&](long long q, bool act, int kk) {
-        double s = 0.0;
-        if (act) {
+    // one step a component and tile: its pair of blocks is loaded while the step before sums
+    RowPair<W> R;
+    double x[27][2];   // the solution at the node and its neighbours
+    double b0 = 0.0, b1 = 0.0, r0 = 0.0;
+    // this step's tile (none yet), component, row and level, and the next step's
+    int tile = ntiles, comp = 1, kk = 0, ncomp = 0, nk = 0;
+    bool act = false, nact = false;
+    int next = find(blockIdx.x, nact, nk);
+#pragma unroll 1
+    while (tile < ntiles || next < ntiles) {
+        const bool have = tile < ntiles;
+        const int q = tile * 64 + lane, count = 27 * min(64, g.nn - tile * 64);
+        if (have) {
+            const size_t o = (size_t)27 * 64 * tile;
+            if (comp == 0 && act) {
+                // unconditional loads, a level inside the column for one outside
 #pragma unroll
-            for (int m = 0; m < 27; ++m) {
-                const int iA = m % 3 - 1, jA = (m / 3) % 3 - 1, kA = m / 9 - 1;
-                if (kk + kA < 0 || kk + kA >= g.nz) continue;
-                const long long qn = q + kA + iA * cst + jA * rst;
-                s = s + SA[27 * lane + m] * xu[qn] + SB[27 * lane + m] * xv[qn];
+                for (int kA = -1; kA <= 1; ++kA) {
+                    if (kA != 0 && g.nz == 1) continue;
+                    const int qk = q + (kk + kA >= 0 && kk + kA < g.nz ? kA : 0);
+#pragma unroll
+                    for (int h = 0; h < 9; ++h) {
+                        const int qn = qk + (h % 3 - 1) * cst + (h / 3 - 1) * rst;
+                        x[9 * kA + 9 + h][0] = xu[qn];
+                        x[9 * kA + 9 + h][1] = xv[qn];
+                    }
+                }
+                b0 = bu[q];
+                b1 = bv[q];
+            }
+            pair_stage<W>(R, (comp ? Avu : Auu) + o, (comp ? Avv : Auv) + o, count, SA, SB, lane);
+        }
+        if (next < ntiles) {
+            const size_t o = (size_t)27 * 64 * next;
+            pair_load<W>(R, (ncomp ? Avu : Auu) + o, (ncomp ? Avv : Auv) + o, 27 * min(64, g.nn - next * 64), lane);
+        }
+        __syncthreads();
+        if (have) {
+            double s = 0.0;
+            if (act) {   // slots in indxA order
+#pragma unroll
+                for (int kA = -1; kA <= 1; ++kA) {
+                    if (kA != 0 && g.nz == 1) continue;
+                    const bool in = kk + kA >= 0 && kk + kA < g.nz;
+                    double t = s;
+#pragma unroll
+                    for (int m = 9 * kA + 9; m < 9 * kA + 18; ++m)
+                        t = t + SA[27 * lane + m] * x[m][0] + SB[27 * lane + m] * x[m][1];
+                    s = in ? t : s;
+                }
+                s -= comp ? b1 : b0;
+            }
+            if (q < g.nn) (comp ? rv : ru)[q] = s;
+            if (comp == 0) {
+                r0 = s;
+            } else if (act) {
+                acc[0] += r0 * r0 + s * s;
+                acc[1] += b0 * b0 + b1 * b1;
             }
         }
-        return s;
-    };
-    int tile = find(blockIdx.x);
-    if (tile < ntiles) pair_load<W>(R, Auu, Auv, (long long)tile * 64, count_of(tile), lane);
-    while (tile < ntiles) {
-        const long long q = (long long)tile * 64 + lane;
-        const bool act = row;
-        const int kk = k;
-        pair_stage<W>(R, SA, SB, lane);
-        pair_load<W>(R, Avu, Avv, (long long)tile * 64, count_of(tile), lane);
         __syncthreads();
-        const double su = product(q, act, kk);
-        __syncthreads();
-        pair_stage<W>(R, SA, SB, lane);
-        const int next = find(tile + gridDim.x);
-        if (next < ntiles) pair_load<W>(R, Auu, Auv, (long long)next * 64, count_of(next), lane);
-        __syncthreads();
-        const double sv = product(q, act, kk);
-        __syncthreads();
-        double r0 = 0.0, r1 = 0.0;
-        if (act) {
-            const double b0 = bu[q], b1 = bv[q];
-            r0 = su - b0;
-            r1 = sv - b1;
-            acc[0] += r0 * r0 + r1 * r1;
-            acc[1] += b0 * b0 + b1 * b1;
-        }
-        if (q < g.nn) {
-            ru[q] = r0;
-            rv[q] = r1;
-        }
         tile = next;
+        act = nact;
+        kk = nk;
+        comp = ncomp;
+        if (ncomp && next < ntiles) next = find(next + gridDim.x, nact, nk);
+        ncomp ^= 1;
     }
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -234,15 +258,18 @@ __global__ __launch_bounds__(NOALLOC_THREADS) void k_resvec_norms(int nb, const 
     s[0][threadIdx.x] = a;
     s[1][threadIdx.x] = b;
     __syncthreads();
-    for (int w = NOALLOC_THREADS / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            s[0][threadIdx.x] += s[0][threadIdx.x + w];
-            s[1][threadIdx.x] += s[1][threadIdx.x + w];
-        }
-        __syncthreads();
+    if (threadIdx.x >= 64) return;
+    // a tree of halves: 128 and 64 apart, then within the wave
+    const int t = threadIdx.x;
+    double v[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        v[c] = (s[c][t] + s[c][t + 128]) + (s[c][t + 64] + s[c][t + 192]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[c] += __shfl_down(v[c], off, 64);
     }
-    if (threadIdx.x == 0) {
-        const double L2 = sqrt(s[0][0]), rhs = sqrt(s[1][0]);
+    if (t == 0) {
+        const double L2 = sqrt(v[0]), rhs = sqrt(v[1]);
         norms[0] = L2;
         norms[1] = rhs > 0.0 ? L2 / rhs : 0.0;
     }
@@ -274,8 +301,7 @@ extern "C" int cism_compute_residual_vector_3d_noalloc(int nx, int ny, int nz, i
     HIP_TRY(hipSetDevice(device));
     double *part = nullptr;
     CISM_TRY(scratch_on_device(device, &part));
-    FGrid g;
-    g.nz = nz; g.sx = nx - 1; g.sy = ny - 1; g.nn = nn;
+    FGrid g{nz, nx - 1, ny - 1, 0, 0, 0, 0, (int)nn, FastDiv((unsigned)nz), FastDiv((unsigned)(nx - 1))};
     // parallel_slap.F90:661-673 (0-based): outflow domains own the west/south boundary rows
     g.ilo = (periodic ? 3 : 2) - 1;
     g.jlo = (periodic ? 3 : 2) - 1;

@@ -59,3 +59,37 @@ def test_residual_tiles(nx, ny, nz, periodic, active, off):
     w2 = np.sqrt((wu ** 2).sum() + (wv ** 2).sum())
     b2 = np.sqrt(((bu ** 2 + bv ** 2) * own).sum())
     assert abs(L2 - w2) <= 1e-13 * w2 and abs(L2r - w2 / b2) <= 1e-13 * w2 / b2
+
+
+@pytest.mark.parametrize("nx,ny,nz", [
+    (304, 264, 1),     # one level: the middle nine slots alone
+    (160, 140, 5),     # 1726 tiles, all but a few without a row, more than one pass of the workgroups
+    (12, 9, 150),      # a tile inside a column
+])
+def test_few_rows_far_apart(nx, ny, nz):
+    """the first and the last owned column alone, blocks that hold NaN where no row reads"""
+    rng = np.random.default_rng(nz)
+    s3, s2 = (nz, nx - 1, ny - 1), (nx - 1, ny - 1)
+    A = [np.asfortranarray(rng.standard_normal((27,) + s3)) for _ in range(4)]
+    bu, bv, u, v = (np.asfortranarray(rng.standard_normal(s3)) for _ in range(4))
+    av = np.zeros(s2, np.int32, order="F")
+    av[2, 2] = av[nx - 3, ny - 3] = 1
+    hip, L = Hip(), G.lib()
+    f = L.cism_compute_residual_vector_3d_noalloc
+    f.argtypes = [C.c_int] * 5 + [C.c_void_p] * 13
+    wu, wv, own = reference(nx, ny, nz, 1, av, A, bu, bv, u, v)
+    for a in A:
+        a[:9, 0] = np.nan          # the level above the surface and the one below the bed
+        a[18:, nz - 1] = np.nan
+        a[:, :, av == 0] = np.nan
+    dev = [hip.put(a) for a in (*A, bu, bv, u, v)]
+    nn = u.size
+    ru, rv, norms = (hip.put(np.full(n, np.nan)) for n in (nn, nn, 2))
+    assert f(nx, ny, nz, 1, 0, None, hip.put(av), *dev, ru, rv, norms) == 0
+    got = [hip.get(p, nn).reshape(s3, order="F") for p in (ru, rv)]
+    L2 = hip.get(norms, 2)[0]
+    hip.free()
+    assert own.sum() == 2
+    assert np.array_equal(got[0], wu) and np.array_equal(got[1], wv)
+    w2 = np.sqrt((wu ** 2).sum() + (wv ** 2).sum())
+    assert abs(L2 - w2) <= 1e-13 * w2
