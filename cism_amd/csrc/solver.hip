@@ -2081,12 +2081,14 @@ int launch_cg_matvec(cism_ctx *c, int which) {
     return CISM_OK;
 }
 
-// one launch of the FP32 fused Chron-Gear update with the column preconditioner, as the
-// inner solves issue it (vectors, factors and scalars of the last mixed solve)
+// one launch of the FP32 fused Chron-Gear update with the column preconditioner, in the form
+// that the inner solves of this grid issue (vectors, factors and scalars of the last mixed
+// solve): with scalars of its own, from the 64 sums that a grid's records always go through
+// (their number is a multiple of 1024), or read from memory
 int launch_cg_update32(cism_ctx *c) {
     CGVecs<float> v = {c->x32, c->b32, c->r32, c->d32, c->z32, c->q32, c->Az32, c->F32, nullptr};
-    const RedSrc src = {nullptr, 0, 0};   // the scalars of the last iteration
-    return launch_cg_update<float>(c, 2, v, src, 0, 0, 1, 1);
+    const RedSrc groups = {c->red_groups, RED_GROUPS, 1}, none = {nullptr, 0, 0};
+    return launch_cg_update<float>(c, 2, v, sia_blocks(c->g) <= CG_FUSE_BLOCKS ? groups : none, 0, 0, 1, 1);
 }
 
 // sums[0] = |x - xref|^2, sums[1] = |xref|^2 over owned nodes

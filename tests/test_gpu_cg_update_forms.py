@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from cism_amd import gpu as G
+from cism_amd import configs, gpu as G
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +82,18 @@ def test_update_forms(n, tiles, nz, precond):
             err = np.linalg.norm(g - w) / np.linalg.norm(w)
             print(f"  {t}: rel L2 diff {err:.2e}")
             assert err < 1e-11
+
+
+@pytest.mark.parametrize("n", [40, 364])   # 29 and 2105 workgroups of 64 columns
+def test_timed_update_leaves_solves_alone(n):
+    """the timing of the FP32 update, in the form that the grid's solves run, between two solves"""
+    p = configs.grf_sheet(ewn=n, nsn=n, nz=3, seed=2)
+    print(f"[cg update] timing {n}x{n}x3", flush=True)
+    with G.Context.for_problem(p) as ctx:
+        lu, lv = ctx.loads(p)
+        solve = lambda: ctx.velo_higher_solve_3d(p, lu, lv, precision=1, maxiter_nonlinear=2)   # noqa: E731
+        first = solve()
+        assert ctx.time_kernel(4, 3) > 0.0
+        again = solve()
+    assert first["fp32_matvecs"] == again["fp32_matvecs"] > 0
+    assert np.array_equal(first["uvel"], again["uvel"]) and np.array_equal(first["vvel"], again["vvel"])
