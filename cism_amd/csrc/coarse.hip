@@ -525,6 +525,7 @@ __global__ __launch_bounds__(16 * CG_TAIL) void k_cg_tail(CgTail T) {
     const int t = threadIdx.x, P = t >> 4, sub = t & 15;
     const CoarseLevel &C = T.lev[NL];
     const int n = 2 * C.ax * C.ay;
+    constexpr int LAST = NL > 0 ? NL - 1 : 0;   // of the smoothed levels
     float4 B[NL > 0 ? NL : 1][9];
     float2 r[NL > 0 ? NL : 1], e[NL > 0 ? NL : 1], dl[NL > 0 ? NL : 1];
     int ci[NL > 0 ? NL : 1], cj[NL > 0 ? NL : 1], c[NL > 0 ? NL : 1];   // this lane's child (c < 0: none)
@@ -568,10 +569,10 @@ __global__ __launch_bounds__(16 * CG_TAIL) void k_cg_tail(CgTail T) {
         }
         __syncthreads();
         if (l + 1 < NL) {   // the next level's residual to its lanes, its pre-smoothed e in its place
-            if (c[NL - 1] >= 0) {
-                r[NL - 1] = x1[c[NL - 1]];
-                e[NL - 1] = make_float2(dl[NL - 1].x * r[NL - 1].x, dl[NL - 1].y * r[NL - 1].y);
-                x1[c[NL - 1]] = e[NL - 1];   // each entry has one lane
+            if (c[LAST] >= 0) {
+                r[LAST] = x1[c[LAST]];
+                e[LAST] = make_float2(dl[LAST].x * r[LAST].x, dl[LAST].y * r[LAST].y);
+                x1[c[LAST]] = e[LAST];   // each entry has one lane
             }
             __syncthreads();
         }

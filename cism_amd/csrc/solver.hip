@@ -188,9 +188,6 @@ static RedSrc red_source(cism_ctx *c, const double *part, int nb) {
     return {c->red_groups, RED_GROUPS, 1};
 }
 
-// the dot products of a Chron-Gear matvec for the update that follows (of nblk workgroups)
-static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop);
-
 // Chron-Gear's scalars from rho = s0 and delta = s1 (pcg:1390-1405, 1501-1512).  zero_stop
 // (inner solves): an exactly zero residual ends the iteration (alpha = 0).
 __device__ inline CgState cg_step(CgState st, double s0, double s1, int first, int zero_stop) {
@@ -1319,7 +1316,6 @@ __global__ __launch_bounds__(CISM_BLOCK) void k_cg_update_level(GridDev g, T *z,
                                                                 DevScal *__restrict__ sc, int cur, int first,
                                                                 int zero_stop, const int32_t *__restrict__ av,
                                                                 const T *__restrict__ F) {
-    using V2 = typename Vec2<T>::t;
     const long long ncol = (long long)g.sx * g.sy;
     const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool solve = q < ncol && av[q];
@@ -1386,6 +1382,7 @@ static inline bool update_level(const GridDev &g, int precond) {
 // nz = 1 with 4,145 workgroups (64 columns each): 190 ms a solve against 201 ms adding them
 // itself; with 1,036 (256 columns each): 138 against 136; 163 x 163 x 21, 415: 523 against 518.
 #define CG_FUSE_BLOCKS 2048
+// the dot products of a Chron-Gear matvec for the update that follows (of nblk workgroups)
 static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop) {
     const RedSrc src = red_source<2>(c, part, nb);
     if (nblk <= CG_FUSE_BLOCKS) return src;
@@ -1405,10 +1402,11 @@ static int launch_cg_update(cism_ctx *c, int precond, CGVecs<T> &v, const RedSrc
             if (precond == PRECOND_SIA_COARSE) cs = c->coarse->colsum;
         const int32_t *um = cs && c->dirichlet_any ? c->umask : nullptr;
         const int32_t *vm = cs && c->dirichlet_any ? c->vmask : nullptr;
-        if (update_level<T>(g, precond))
-            hipLaunchKernelGGL(k_cg_update_level<T>, dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0, c->stream, g, v.z,
-                               v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F);
-        else {
+        if (update_level<T>(g, precond)) {
+            if constexpr (std::is_same<T, double>::value)
+                hipLaunchKernelGGL(k_cg_update_level<T>, dim3(nblocks_for(g.nn)), dim3(CISM_BLOCK), 0, c->stream, g,
+                                   v.z, v.Az, v.d, v.q, v.x, v.r, src, c->sc, cur, first, zero_stop, c->av, v.F);
+        } else {
             auto kern = g.nz <= 12   ? (src.n ? k_cg_update_sia<T, 12, true> : k_cg_update_sia<T, 12, false>)
                         : g.nz <= 24 ? (src.n ? k_cg_update_sia<T, 24, true> : k_cg_update_sia<T, 24, false>)
                                      : (src.n ? k_cg_update_sia<T, 48, true> : k_cg_update_sia<T, 48, false>);
@@ -1437,7 +1435,7 @@ template <typename T, typename M>
 static int run_cg(cism_ctx *c, const M A, CGVecs<T> v, int chrongear, int precond, int maxiters,
                   double tol, int check, double *err_out, int *niters_out, int x_zero = 0) {
     const GridDev &g = c->g;
-    const int nb = red_blocks_for(g.nn), nbm = nblocks_for(g.nn), nb2 = nblocks_for(2 * g.nn);
+    const int nb = red_blocks_for(g.nn), nbm = nblocks_for(g.nn);
     const int nbv = M::xcd ? xcd_blocks_for(g.nn) : nbm;   // matvec grid
     const unsigned chunk = xcd_chunk_for(g.nn);
     const int nbr = M::slots ? xcd_slots_for(g.nn) : nbm;   // partials of a matvec
