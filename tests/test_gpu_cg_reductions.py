@@ -1,9 +1,10 @@
 """The dot products that the PCG kernels add for themselves, at the sizes where their form
 changes: one record a group (up to 64 node blocks), up to eight (512), more (a launch of its
-own), and updates of more than 2048 workgroups, whose scalars come from one workgroup.  A dozen
-iterations from the same start against the oracle, as in test_gpu_parity.test_pcg_short: only
-the order of the global sums differs, so the iterates agree to rounding (1e-11).  Twelve
-iterations end between two convergence checks, eleven leave a standard PCG's halo as it is."""
+own, from 513 on), and updates of more than 2048 workgroups, whose scalars come from one
+workgroup.  A dozen iterations from the same start against the oracle, as in
+test_gpu_parity.test_pcg_short: only the order of the global sums differs, so the iterates agree
+to rounding (1e-11).  Twelve iterations end between two convergence checks, eleven leave a
+standard PCG's halo as it is."""
 import numpy as np
 import pytest
 
@@ -17,8 +18,9 @@ SIZES = {                                # nodes nz (ewn + 3) (nsn + 3) in block
     "64_blocks": (61, 61, 4),
     "65_blocks": (62, 61, 4),
     "512_blocks": (125, 125, 8),
-    "513_blocks": (126, 125, 8),
-    "1040_update_blocks": (254, 256, 2),
+    "513_blocks": (190, 167, 4),
+    "516_blocks": (126, 125, 8),
+    "1041_update_blocks": (254, 256, 2),
     "2105_update_blocks": (364, 364, 2),
 }
 
@@ -27,6 +29,9 @@ SIZES = {                                # nodes nz (ewn + 3) (nsn + 3) in block
 def system(request):
     ewn, nsn, nz = SIZES[request.param]
     p = configs.grf_sheet(ewn=ewn, nsn=nsn, nz=nz, seed=8)
+    blocks = -(-nz * (ewn + 3) * (nsn + 3) // 256)
+    columns = -(-(ewn + 3) * (nsn + 3) // 64)
+    assert str(columns if "update" in request.param else blocks) == request.param.split("_")[0]
     return (p,) + assembled_system(p, seed=5)[:5]
 
 
