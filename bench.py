@@ -293,7 +293,8 @@ def main(argv=None):
     gbs64 = bytes64 / (ms64 * 1e-3) / 1e9
     n_el = int(p.active_cell.sum()) * (p.nz - 1)
     asm_tflops = n_el * FLOP_PER_ELEMENT / (ms_asm * 1e-3) / 1e12
-    traffic = measured_traffic(a.workload)
+    matvec32 = "k_matvec_dots<float, MatSym32>"
+    traffic = measured_traffic(a.workload, matvec32)
 
     cpu = cpu_all = None
     if not a.no_cpu_baseline:
@@ -361,7 +362,7 @@ def main(argv=None):
                      "frac_fp64_peak": round(asm_tflops / FP64_VALU_PEAK_TFLOPS, 4)},
         "roofline": {"bound": "hbm", "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs32 / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_matvec_dots<float, MatSym32>",
+                     "kernel": matvec32,
                      "algorithmic_bytes_per_launch": bytes32},
         "cpu_baseline": cpu,
         "cpu_baseline_all_cores": cpu_all,
@@ -412,17 +413,20 @@ def inputs_hash(p):
     return h.hexdigest()[:16]
 
 
-def measured_traffic(workload_name):
+def measured_traffic(workload_name, kernel):
     """HBM bytes per launch of the FP32 matvec from the committed rocprofv3 --pmc summary of
     this workload (FETCH_SIZE + WRITE_SIZE, each scaled by the copy-kernel calibration), or
-    None when no such summary exists."""
+    None when no such summary exists or it was taken on another kernel than the one named."""
     path = os.path.join(ROOT, "profiles", f"pmc_k_matvec_dots_fp32_{workload_name}.txt")
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        for line in f:
-            if line.startswith("traffic_bytes_per_launch:"):
-                return int(float(line.split(":", 1)[1]))
+        lines = f.read().splitlines()
+    if not any(ln.startswith(f"kernel: void {kernel}(") for ln in lines):
+        return None
+    for ln in lines:
+        if ln.startswith("traffic_bytes_per_launch:"):
+            return int(float(ln.split(":", 1)[1]))
     return None
 
 

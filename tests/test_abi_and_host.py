@@ -63,6 +63,20 @@ def test_no_standard_pcg_on_the_fp32_matrix():
     assert not [n for n in kernels if "MatSym32" in n]
 
 
+def test_bench_traffic_is_of_the_reported_kernel(tmp_path, monkeypatch):
+    """the bench line's traffic comes from a counter summary of the kernel it names"""
+    import bench
+    kernel = "k_matvec_dots<float, MatSym32>"
+    src = os.path.join(ROOT, "profiles", "pmc_k_matvec_dots_fp32_c5.txt")
+    assert bench.measured_traffic("c5", kernel) > 0
+    os.makedirs(tmp_path / "profiles")
+    text = open(src).read()
+    for other, want in ((kernel, True), ("k_matvec_dots<float, 2, MatSym32>", False)):
+        (tmp_path / "profiles" / os.path.basename(src)).write_text(text.replace(kernel, other))
+        monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+        assert (bench.measured_traffic("c5", kernel) is not None) == want
+
+
 def test_fortran_shim_exports():
     path = os.path.join(ROOT, "cism_amd", "libcism_fortran.so")
     if not os.path.exists(path):
