@@ -64,8 +64,8 @@ __host__ __device__ inline long long keidx(int ent, long long e) {
 // An element's eight records are padded to 194 doubles: the eight elements a wave reads
 // side by side then start in eight disjoint groups of four banks.  The nodes' (x, y, z, u,
 // v) share the records' memory (a barrier separates their last read from the first
-// record store), which keeps the workgroup under 26.7 KB: six workgroups (three waves per
-// SIMD) fit a CU.
+// record store).  With the validity flags and the word that __syncthreads_or keeps a workgroup
+// has 27,200 bytes, 27,648 as allocated: five workgroups (ten waves) fit a CU.
 #define QP_REC 24
 #define EL_REC (8 * QP_REC + 2)
 struct QPLds {
@@ -76,7 +76,8 @@ struct QPLds {
     double f[EL_ELEM][8];
     double ev[EL_ELEM][8];
 };
-static_assert(sizeof(QPLds) + EL_ELEM * sizeof(int) <= 163840 / 6, "six element workgroups per CU");
+static_assert(5 * ((sizeof(QPLds) + EL_ELEM * sizeof(int) + 256 + 511) / 512 * 512) <= 163840,
+              "five element workgroups per CU");
 
 // One quadrature point p of a hexahedral element whose 8 nodes are given as
 // (x, y, z, u, v) records: basis-function derivatives (get_basis_function_

@@ -121,7 +121,8 @@ __global__ void k_reduce_final(const double *__restrict__ groups, int mode, DevS
 // are then 64 records with chunk 1.  With nz = 1, 124 x 136 columns (66 records) the two
 // launches took 2.7 + 4.1 us and two launch gaps of every iteration's 25 us; here the sums
 // take about 1 us of the update kernel.  The line lies at 512 records: each workgroup reads
-// them all from L2, 8 KB, which 2,000 workgroups still do in the time of one launch.
+// them all from L2, 8 KB, which 2,000 workgroups still do in the time of one launch.  The FP32
+// matvec's records, in xcd_slots_for places, a multiple of 1024, always take the extra launch.
 #define RED_CHUNK 8
 struct RedSrc {
     const double *p;
@@ -438,7 +439,7 @@ int launch_matvec64(cism_ctx *c, const double *A, const double *x, double *y) {
 // y = A x plus per-block partial dot products over owned nodes, s0 = (r, x), s1 = (y, x)
 // (Chron-Gear's (r, z), (Az, z)).  One lane per node, one pass over the grid.
 // FP64, 163 x 163 x 21: 74.2 us with chunks of 128 blocks, 64.1 us with chunks of equal number
-// for every XCD (xcd_chunk_for); 35 x 35 x 10, 46 blocks, 5.9 -> 5.7 us.
+// for every XCD (xcd_chunk_for); 34 x 34 x 10, 46 blocks, 5.9 -> 5.7 us.
 template <typename T, typename M>
 __global__ __launch_bounds__(CISM_BLOCK) void k_matvec_dots(GridDev g, unsigned chunk, const M A,
                                                             const int32_t *__restrict__ av,
@@ -923,7 +924,7 @@ int launch_halo_mat(cism_ctx *c, double *A) {
 // same operations on the same values as a pass over d, a halo copy and a matvec.  The
 // second launch updates x and r, and with the diagonal or no preconditioner forms the next
 // z and the partials of (r, z) too.  Both form their scalar from the partials they need
-// (red_sums).  35 x 35 x 10, diagonal preconditioner: an iteration was 10 launches of 2.4 to
+// (red_sums).  34 x 34 x 10, diagonal preconditioner: an iteration was 10 launches of 2.4 to
 // 6 us, 42 us in all (187 ms a solve); two take 7.9 + 4.1 us (88 ms a solve, checks included).
 
 // beta = (r, z) / the last (r, z)   (pcg:366-382)
@@ -947,7 +948,7 @@ __device__ inline CgState std_alpha_step(CgState st, double s0) {
 // direction, which are then the shorter of the two.  The windows' z and d are on their way
 // while the scalar is formed.  Bound: at small sizes the latency of the scalar and of three
 // groups of matrix loads in one wave per SIMD, at large ones the matrix from past L2.  Formed
-// 27 times a node instead: 12.0 us at 35 x 35 x 10 (7.9 here); an iteration at 31 x 31 x 10
+// 27 times a node instead: 12.0 us at 34 x 34 x 10 (7.9 here); an iteration at 31 x 31 x 10
 // 14.2 us (10.0), 120 x 130 x 11 61 us (53), 400 x 410 x 11 453 us (391), 400 x 410 x 2 103 us
 // (89), 40 x 40 x 60 40 us (33).
 #define STD_AHEAD 4   // entries per lane loaded ahead: all of three windows to 41 levels
@@ -1378,9 +1379,15 @@ static inline bool update_level(const GridDev &g, int precond) {
 }
 
 // An update of more workgroups than this takes its scalars from one workgroup launched before
-// it: every workgroup of the update would wait for the records again.  515 x 515 columns at
-// nz = 1 with 4,145 workgroups (64 columns each): 190 ms a solve against 201 ms adding them
-// itself; with 1,036 (256 columns each): 138 against 136; 163 x 163 x 21, 415: 523 against 518.
+// it: every workgroup of the update would wait for the records again.  Linear part of a solve, a
+// launch before it / scalars of its own:
+//   one level, FP64 (256 columns a workgroup): 1,239 workgroups 20.9 / 19.6 ms, 1,931 28.1 / 27.0,
+//     2,275 32.4 / 31.4, 3,930 55.1 / 54.0
+//   FP64, 64 columns a workgroup, 11 or 21 levels: 1,165 33.6 / 33.2 ms, 1,839 98.8 / 97.7, 2,538
+//     133.9 / 132.9, 3,954 104.4 / 104.8
+//   mixed precision, 11 levels: 1,165 15.9 / 16.3 ms, 1,839 41.4 / 40.9, 3,067 40.2 / 40.6, 3,954
+//     56.3 / 56.9
+// so the line divides what the mixed solves lose past it from what one level still gains.
 #define CG_FUSE_BLOCKS 2048
 // the dot products of a Chron-Gear matvec for the update that follows (of nblk workgroups)
 static RedSrc cg_source(cism_ctx *c, const double *part, int nb, int nblk, int cur, int first, int zero_stop) {

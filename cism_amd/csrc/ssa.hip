@@ -323,9 +323,10 @@ __device__ __forceinline__ double quad_sum(double v) {
 // Four lanes a cell, lane p at quadrature point p: the point's layers and element terms are one
 // lane's work, the sums over the points are quad sums in point order (the values of one lane
 // that runs the points in turn), and the layer fields leave through LDS in contiguous runs.
-// Bound: the FP64 powers and divisions, 40 of each a cell and 10 layers.  A lane per cell left
-// one wave a SIMD and each layer field in steps of 80 to 320 bytes: DIVA, 516 x 516 cells, 10
-// layers 546 us, 199 here.
+// Bound: the FP64 powers and divisions, of DIVA 40 and 120 a cell and 10 layers (a power a point
+// and layer, two divisions by the old viscosity and one for omega).  A lane per cell left one
+// wave a SIMD and each layer field in steps of 80 to 320 bytes: DIVA, 516 x 516 cells, 10 layers
+// 546 us, 199 here.
 #define DEPTH_CELLS 64   // cells a workgroup
 template <int APPROX>
 __global__ __launch_bounds__(256) void k_element_depth(GridDev g, DepthDev d, const int32_t *__restrict__ ac,
